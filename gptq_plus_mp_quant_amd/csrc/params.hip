@@ -68,90 +68,309 @@ __global__ __launch_bounds__(256) void k_find_params(const TW* __restrict__ w, i
 // then a maxshrink*grid x maxshrink*grid shrink grid over (xmin, xmax); each candidate's row
 // error sum |q - x|^norm is reduced in a fixed order and the first strict minimum wins
 // (clip_zero = 0: the groupwise search of :354-386, from the group's own min / max).
-// One 256-thread workgroup per (row, group).
-template <typename TW>
-__global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ w, int R, int C,
-                                                         int64_t ldw, int gs, float maxq, int sym,
-                                                         int clip_zero, float norm, int grid, int steps,
-                                                         float* __restrict__ scale,
-                                                         float* __restrict__ zero) {
-  __shared__ float red[256];
-  __shared__ float red2[256];
-  const int tid = threadIdx.x;
-  const int r = blockIdx.x, grp = blockIdx.y;
-  const int c0 = grp * gs;
-  const int c1 = min(C, c0 + gs);
-  const TW* row = w + (int64_t)r * ldw;
-  float mn = __builtin_inff(), mx = -__builtin_inff();
-  for (int c = c0 + tid; c < c1; c += 256) {
-    const float v = rq_load_elem(row + c);
-    mn = rq_nan_min(mn, v);
-    mx = rq_nan_max(mx, v);
-  }
-  red[tid] = mn;
-  red2[tid] = mx;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (tid < o) {
-      red[tid] = rq_nan_min(red[tid], red[tid + o]);
-      red2[tid] = rq_nan_max(red2[tid], red2[tid + o]);
+//
+// Bound by VALU issue: a candidate costs every element a divide, a round, a clamp and a power.
+//  - Symmetric: s depends on (i, j) only through max(|xmin1|, xmax1), one of 2 * steps values, and
+//    equal steps have equal errors, so 2 * steps candidates are evaluated instead of steps^2
+//    (50 instead of 625 at the default grid).
+//  - x / s with s shared by all elements: y = RN(1 / s), q0 = RN(x y), then one residual step
+//    q0 + y (x - s q0) in two fused operations is the correctly rounded quotient (Markstein)
+//    while nothing underflows; steps outside [2^-60, 2^60] take the IEEE divide.
+//  - |q - x|^norm in 64-bit arithmetic (mse_pow), a quarter of powf's instructions and closer to
+//    the exact power.
+//  - One wave per candidate batch: a lane holds 4 of 256 interleaved partial sums, and 8
+//    candidates are reduced together by halving exchanges (10 shuffles instead of 48), with no
+//    barrier.  Up to MSE_WIDE elements a wave owns one (row, group); wider rows share a
+//    workgroup's 4 waves, which take every fourth batch.
+// 1024 x 4096 fp32 against one 256-thread workgroup per (row, group), every candidate, the IEEE
+// divide and powf: symmetric 16.3 -> 0.43 ms (128-column groups) and 10.7 -> 0.34 ms (per row),
+// asymmetric 16.5 -> 4.2 and 10.5 -> 3.0 ms.
+constexpr int MSE_WIDE = 1024;          // above: one (row, group) per workgroup
+constexpr int MSE_LDS_MAX = 16384;      // elements staged in LDS; wider groups are read in place
+constexpr int MSE_B = 8;                // candidates per batch
+
+struct MseLog {
+  double inv, log2c;                    // 1 / c and log2(c) of an interval's centre c
+};
+
+// |d|^p for d >= 0 finite and p > 0, in 64 bits and rounded once: log2(d) = e + log2(c) +
+// log2(m / c) with m / c - 1 within 0.0304 of 0 (a table of 16 centres c), 2^y by its
+// fractional part; both polynomials are near-minimax (2^-36 and 2^-34), so the result is within
+// 0.5 + 2^-9 units of the last place (powf: 1).
+__device__ __forceinline__ float mse_pow(float d, double p, const MseLog* tab) {
+  const float m = __builtin_amdgcn_frexp_mantf(d);
+  const int e = __builtin_amdgcn_frexp_expf(d);
+  const MseLog t = tab[(__float_as_uint(m) >> 19) & 15];
+  const double r = __builtin_fma((double)m, t.inv, -1.0);
+  double a = 0x1.27c1ba5fe9d34p-2;
+  a = __builtin_fma(a, r, -0x1.719d5484e3a26p-2);
+  a = __builtin_fma(a, r, 0x1.ec70971caf89bp-2);
+  a = __builtin_fma(a, r, -0x1.7154742aec3edp-1);
+  a = __builtin_fma(a, r, 0x1.71547652bdc8bp+0);
+  const double y = p * __builtin_fma(a, r, (double)e + t.log2c);
+  const double n = __builtin_rint(y);
+  const double f = y - n;
+  double z = 1.531008147539287e-05;
+  z = __builtin_fma(z, f, 0.00015469731991027595);
+  z = __builtin_fma(z, f, 0.001333345055956001);
+  z = __builtin_fma(z, f, 0.009618025602929684);
+  z = __builtin_fma(z, f, 0.055504109412156666);
+  z = __builtin_fma(z, f, 0.2402265121359518);
+  z = __builtin_fma(z, f, 0.6931471805459303);
+  z = __builtin_fma(z, f, 0.9999999999595488);
+  const float v = (float)__builtin_amdgcn_ldexp(z, (int)n);
+  return d == 0.0f ? 0.0f : v;
+}
+
+// The step and zero of candidate c, and whether it is one of the grid's.  Symmetric candidates:
+// c < steps is |xmin| shrunk by row c of the grid (where some column leaves xmax no larger), the
+// others xmax shrunk by column c - steps.
+struct MseGrid {
+  float xmin, xmax, maxq;
+  int sym, grid, steps, n;
+  __device__ __forceinline__ float fac(int i) const { return (float)(1.0 - (double)i / (double)grid); }
+  __device__ __forceinline__ float lo(int i) const { return fabsf(fac(i) * xmin); }
+  __device__ __forceinline__ float hi(int j) const { return fac(j) * xmax; }
+  __device__ __forceinline__ bool params(int c, float* s, float* z) const {
+    if (sym) {
+      const int k = c < steps ? c : c - steps;
+      const float m = c < steps ? lo(k) : hi(k);
+      // the other side's smallest value decides whether max() ever takes m
+      const float other = c < steps ? rq_nan_min(hi(0), hi(steps - 1)) : lo(steps - 1);
+      *s = rq_clamp_min(m, 1e-5f) / maxq;
+      *z = 0.0f;
+      return c < n && !(other > m);
     }
+    const float xmin1 = fac(c / steps) * xmin, xmax1 = fac(c % steps) * xmax;
+    *s = (xmax1 - xmin1) / maxq;
+    *z = __builtin_rintf(-xmin1 / *s);
+    return c < n;
+  }
+  // place of candidate c in the search order (row by row), for equal errors
+  __device__ int first(int c) const {
+    if (!sym) return c;
+    const bool row = c < steps;
+    const int k = row ? c : c - steps;
+    const float m = row ? lo(k) : hi(k);
+    int o = 0;
+    while (o < steps - 1 && (row ? hi(o) : lo(o)) > m) ++o;
+    return row ? k * steps + o : o * steps + k;
+  }
+};
+
+// The element's code times the step (the rounded quotient t = x / s comes in).
+template <bool SYM>
+__device__ __forceinline__ float mse_quant(float t, float s, float z, float maxq) {
+  t = __builtin_rintf(t);
+  if (SYM) {
+    t = (t < -(maxq + 1.0f)) ? -(maxq + 1.0f) : t;
+    t = (t > maxq) ? maxq : t;
+    return s * t;
+  }
+  t = t + z;
+  t = (t < 0.0f) ? 0.0f : t;
+  t = (t > maxq) ? maxq : t;
+  return s * (t - z);
+}
+
+// One batch: the partial sums of MSE_B candidates over the lane's elements.
+template <bool SYM, typename TX>
+__device__ __forceinline__ void mse_batch(const TX* x, int n, int lane, const float* s, const float* z, const float* y,
+                                          float maxq, double p, const MseLog* tab, float* part) {
+  float acc[MSE_B][4];
+#pragma unroll
+  for (int k = 0; k < MSE_B; ++k)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[k][u] = 0.0f;
+  for (int c0 = 0; c0 < n; c0 += 256) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (c0 + 64 * u >= n) break;                     // the same for the whole wave
+      const int c = c0 + 64 * u + lane;
+      const bool in = c < n;
+      const float v = rq_load_elem(x + (in ? c : 0));
+#pragma unroll
+      for (int k = 0; k < MSE_B; ++k) {
+        const float q0 = v * y[k];
+        const float t = __builtin_fmaf(__builtin_fmaf(-s[k], q0, v), y[k], q0);
+        const float e = mse_pow(fabsf(mse_quant<SYM>(t, s[k], z[k], maxq) - v), p, tab);
+        acc[k][u] += in ? e : 0.0f;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < MSE_B; ++k) part[k] = (acc[k][0] + acc[k][2]) + (acc[k][1] + acc[k][3]);
+}
+
+// The same for one candidate with any step, norm and data: IEEE divide and powf.
+template <bool SYM, typename TX>
+__device__ __attribute__((noinline)) float mse_any(const TX* x, int n, int lane, float s, float z, float maxq,
+                                                   float norm) {
+  float sum[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    sum[u] = 0.0f;
+    for (int c = 64 * u + lane; c < n; c += 256) {
+      const float v = rq_load_elem(x + c);
+      sum[u] += powf(fabsf(mse_quant<SYM>(v / s, s, z, maxq) - v), norm);
+    }
+  }
+  return (sum[0] + sum[2]) + (sum[1] + sum[3]);
+}
+
+template <bool SYM, typename TW, bool STAGED>
+__global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ w, int R, int C,
+                                                         int64_t ldw, int gs, int ng, float maxq,
+                                                         int clip_zero, float norm, int grid, int steps,
+                                                         int per_wg, float* __restrict__ scale,
+                                                         float* __restrict__ zero) {
+  extern __shared__ __attribute__((aligned(16))) float xs[];
+  __shared__ MseLog tab[16];
+  __shared__ float best_e[4];
+  __shared__ int best_c[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid < 16) {
+    const double c = 0.5 + (tid + 0.5) / 32.0;
+    tab[tid].inv = 1.0 / c;
+    tab[tid].log2c = log2(c);
+  }
+  __syncthreads();
+  // per_wg 4: each wave its own (row, group); per_wg 1: the waves share one.  Grid: rows x groups.
+  const bool shared = per_wg == 1;
+  const int64_t item = shared ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
+  const bool live = item < (int64_t)R * ng;
+  const int r = live ? (int)(item % R) : 0, grp = live ? (int)(item / R) : 0;
+  const int c0 = grp * gs;
+  const int n = live ? min(C, c0 + gs) - c0 : 0;
+  const TW* row = w + (int64_t)r * ldw + c0;
+  float* xw = xs + (shared ? 0 : wave * gs);
+  if (STAGED) {
+    for (int c = shared ? tid : lane; c < n; c += shared ? 256 : 64) xw[c] = rq_load_elem(row + c);
     __syncthreads();
   }
-  float xmin = clip_zero ? rq_nan_min(red[0], 0.0f) : red[0];
-  float xmax = clip_zero ? rq_nan_max(red2[0], 0.0f) : red2[0];
-  if (!sym && xmin == 0.0f && xmax == 0.0f) {
-    xmin = -1.0f;
-    xmax = 1.0f;
+  auto elem = [&](int c) -> float { return STAGED ? xw[c] : rq_load_elem(row + c); };
+  // min and max in the order of 256 interleaved lanes (it decides which of +0 and -0 is kept)
+  float mn[4], mx[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    mn[u] = __builtin_inff();
+    mx[u] = -__builtin_inff();
+    for (int c = 64 * u + lane; c < n; c += 256) {
+      mn[u] = rq_nan_min(mn[u], elem(c));
+      mx[u] = rq_nan_max(mx[u], elem(c));
+    }
   }
-  float bscale, bzero;
-  rq_params_from_minmax(red[0], red2[0], maxq, sym, &bscale, &bzero, clip_zero);
-  float best = __builtin_inff();
-  for (int i = 0; i < steps; ++i) {
-    const float fi = (float)(1.0 - (double)i / (double)grid);
-    for (int j = 0; j < steps; ++j) {
-      const float fj = (float)(1.0 - (double)j / (double)grid);
-      const float xmin1 = fi * xmin, xmax1 = fj * xmax;
-      float s1, z1;
-      if (sym) {
-        s1 = rq_clamp_min(rq_nan_max(fabsf(xmin1), xmax1), 1e-5f) / maxq;
-        z1 = 0.0f;
-      } else {
-        s1 = (xmax1 - xmin1) / maxq;
-        z1 = __builtin_rintf(-xmin1 / s1);
+  float rmin = rq_nan_min(rq_nan_min(mn[0], mn[2]), rq_nan_min(mn[1], mn[3]));
+  float rmax = rq_nan_max(rq_nan_max(mx[0], mx[2]), rq_nan_max(mx[1], mx[3]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    rmin = rq_nan_min(rmin, __shfl_down(rmin, o, 64));
+    rmax = rq_nan_max(rmax, __shfl_down(rmax, o, 64));
+  }
+  rmin = __shfl(rmin, 0, 64);
+  rmax = __shfl(rmax, 0, 64);
+  MseGrid g;
+  g.xmin = clip_zero ? rq_nan_min(rmin, 0.0f) : rmin;
+  g.xmax = clip_zero ? rq_nan_max(rmax, 0.0f) : rmax;
+  if (!SYM && g.xmin == 0.0f && g.xmax == 0.0f) {
+    g.xmin = -1.0f;
+    g.xmax = 1.0f;
+  }
+  g.maxq = maxq;
+  g.sym = SYM;
+  g.grid = grid;
+  g.steps = steps;
+  g.n = SYM ? 2 * steps : steps * steps;
+  const double p = (double)norm;
+  // the lane's own candidate among the batch's: bit 5, 4, 3 of the lane
+  const int mine = ((lane >> 5) & 1) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1);
+  float be = __builtin_inff();
+  int bc = -1;
+  for (int b = shared ? wave : 0; b * MSE_B < g.n; b += shared ? 4 : 1) {
+    // lane k < 8 works out candidate k's step; every lane then reads all eight
+    float cs, cz;
+    const bool ok = g.params(b * MSE_B + (lane & (MSE_B - 1)), &cs, &cz);
+    const float cy = 1.0f / cs;
+    // steps for which the residual divide is exact, and finite data (an infinity or NaN in the
+    // row makes every step one)
+    const bool good = cs >= 0x1p-60f && cs <= 0x1p60f && norm > 0.0f && norm < 64.0f;
+    float s[MSE_B], z[MSE_B], y[MSE_B], part[MSE_B];
+#pragma unroll
+    for (int k = 0; k < MSE_B; ++k) {
+      s[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
+      z[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
+      y[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cy), k));
+    }
+    const uint64_t valid = __ballot(ok) & 255, exact = __ballot(good || !ok) & 255;
+    if (!valid) continue;
+    if (exact == 255) {
+      if (STAGED) mse_batch<SYM>(xw, n, lane, s, z, y, maxq, p, tab, part);
+      else mse_batch<SYM>(row, n, lane, s, z, y, maxq, p, tab, part);
+    } else {
+      for (int k = 0; k < MSE_B; ++k) {
+        const float sk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
+        const float zk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
+        const float v = STAGED ? mse_any<SYM>(xw, n, lane, sk, zk, maxq, norm)
+                               : mse_any<SYM>(row, n, lane, sk, zk, maxq, norm);
+#pragma unroll
+        for (int j = 0; j < MSE_B; ++j)
+          if (j == k) part[j] = v;
       }
-      float part = 0.0f;
-      for (int c = c0 + tid; c < c1; c += 256) {
-        const float x = rq_load_elem(row + c);
-        float q;
-        if (sym) {
-          q = s1 * rq_quant_code(x, s1, -(maxq + 1.0f), maxq);
-        } else {
-          float t = __builtin_rintf(x / s1) + z1;
-          t = (t < 0.0f) ? 0.0f : t;
-          t = (t > maxq) ? maxq : t;
-          q = s1 * (t - z1);
-        }
-        part += powf(fabsf(q - x), norm);
-      }
-      __syncthreads();                  // red[] of the previous candidate fully read
-      red[tid] = part;
-      __syncthreads();
-      for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) red[tid] = red[tid] + red[tid + o];
-        __syncthreads();
-      }
-      const float err = red[0];
-      if (err < best) {                 // same value in every thread: uniform update
-        best = err;
-        bscale = s1;
-        bzero = z1;
+    }
+    // the tree of 64 partial sums (l + (l + 32), + 16, ...), halving the candidates a lane keeps
+    // for the first three levels; each lane ends with the sum of candidate `mine`
+    float h4[4], h2[2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool up = lane & 32;
+      const float keep = up ? part[k + 4] : part[k], send = up ? part[k] : part[k + 4];
+      h4[k] = keep + __shfl_xor(send, 32, 64);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const bool up = lane & 16;
+      const float keep = up ? h4[k + 2] : h4[k], send = up ? h4[k] : h4[k + 2];
+      h2[k] = keep + __shfl_xor(send, 16, 64);
+    }
+    const bool up = lane & 8;
+    float err = (up ? h2[1] : h2[0]) + __shfl_xor(up ? h2[0] : h2[1], 8, 64);
+    err += __shfl_xor(err, 4, 64);
+    err += __shfl_xor(err, 2, 64);
+    err += __shfl_xor(err, 1, 64);
+    const int c = b * MSE_B + mine;
+    if ((valid >> mine) & 1) {
+      if (err < be || (err == be && bc >= 0 && g.first(c) < g.first(bc))) {
+        be = err;
+        bc = c;
       }
     }
   }
-  if (tid == 0) {
-    scale[(int64_t)grp * R + r] = bscale;
-    zero[(int64_t)grp * R + r] = bzero;
+  auto merge = [&](float oe, int oc) {
+    if (oc >= 0 && (bc < 0 || oe < be || (oe == be && oc != bc && g.first(oc) < g.first(bc)))) {
+      be = oe;
+      bc = oc;
+    }
+  };
+#pragma unroll
+  for (int o = 32; o >= 8; o >>= 1) {
+    const float oe = __shfl_xor(be, o, 64);
+    const int oc = __shfl_xor(bc, o, 64);
+    merge(oe, oc);
+  }
+  if (shared) {
+    if (lane == 0) {
+      best_e[wave] = be;
+      best_c[wave] = bc;
+    }
+    __syncthreads();
+    for (int k = 0; k < 4; ++k) merge(best_e[k], best_c[k]);
+  }
+  if (live && lane == 0 && (!shared || wave == 0)) {
+    float bs, bz;
+    if (bc >= 0) g.params(bc, &bs, &bz);
+    else rq_params_from_minmax(rmin, rmax, maxq, SYM, &bs, &bz, clip_zero);
+    scale[(int64_t)grp * R + r] = bs;
+    zero[(int64_t)grp * R + r] = bz;
   }
 }
 
@@ -479,6 +698,29 @@ inline bool launch_gather_rows(const TS* src, int64_t lds, int rows, int C, cons
   return true;
 }
 
+// Groups up to MSE_WIDE elements: a wave each, four per workgroup; wider ones a workgroup each;
+// staged in LDS up to MSE_LDS_MAX elements (64 KB).
+template <typename TW>
+int launch_find_params_mse(const TW* w, int R, int C, int64_t ldw, int gs, int ng, int maxq, int sym, int clip_zero,
+                           float norm, int grid, int steps, float* scale, float* zero, hipStream_t s) {
+  const int width = gs < C ? gs : C;
+  const int per_wg = width <= MSE_WIDE ? 4 : 1;
+  const int64_t items = (int64_t)R * ng, wgs = (items + per_wg - 1) / per_wg;
+  if (wgs > 0x7fffffff || (int64_t)steps * steps > (1 << 28)) return RQ_EINVAL;
+  const bool staged = width <= MSE_LDS_MAX;
+  const size_t lds = staged ? (size_t)per_wg * width * sizeof(float) : 0;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), lds, s, w, R, C, ldw, width, ng, (float)maxq, clip_zero,
+                       norm, grid, steps, per_wg, scale, zero);
+  };
+  if (sym && staged) go(k_find_params_mse<true, TW, true>);
+  else if (sym) go(k_find_params_mse<true, TW, false>);
+  else if (staged) go(k_find_params_mse<false, TW, true>);
+  else go(k_find_params_mse<false, TW, false>);
+  RQ_CHECK_LAUNCH();
+  return RQ_OK;
+}
+
 }  // namespace
 
 extern "C" int rq_find_params(const void* w, int w_dtype, int R, int C, int64_t ldw, int group_size,
@@ -512,20 +754,16 @@ extern "C" int rq_find_params_mse(const void* w, int w_dtype, int R, int C, int6
   const int steps = (int)(maxshrink * grid);   // int(self.maxshrink * self.grid)
   if (steps <= 0) return RQ_EINVAL;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  dim3 g(R, ng), block(256);
   if (w_dtype == RQ_F16)
-    hipLaunchKernelGGL(k_find_params_mse<__half>, g, block, 0, s, (const __half*)w, R, C, ldw, gs,
-                       (float)maxq, sym, clip_zero, (float)norm, grid, steps, scale, zero);
-  else if (w_dtype == RQ_BF16)
-    hipLaunchKernelGGL(k_find_params_mse<__hip_bfloat16>, g, block, 0, s, (const __hip_bfloat16*)w, R,
-                       C, ldw, gs, (float)maxq, sym, clip_zero, (float)norm, grid, steps, scale, zero);
-  else if (w_dtype == RQ_F32)
-    hipLaunchKernelGGL(k_find_params_mse<float>, g, block, 0, s, (const float*)w, R, C, ldw, gs,
-                       (float)maxq, sym, clip_zero, (float)norm, grid, steps, scale, zero);
-  else
-    return RQ_EINVAL;
-  RQ_CHECK_LAUNCH();
-  return RQ_OK;
+    return launch_find_params_mse((const __half*)w, R, C, ldw, gs, ng, maxq, sym, clip_zero, (float)norm, grid, steps,
+                                  scale, zero, s);
+  if (w_dtype == RQ_BF16)
+    return launch_find_params_mse((const __hip_bfloat16*)w, R, C, ldw, gs, ng, maxq, sym, clip_zero, (float)norm,
+                                  grid, steps, scale, zero, s);
+  if (w_dtype == RQ_F32)
+    return launch_find_params_mse((const float*)w, R, C, ldw, gs, ng, maxq, sym, clip_zero, (float)norm, grid, steps,
+                                  scale, zero, s);
+  return RQ_EINVAL;
 }
 
 extern "C" int rq_prepare_subgroup(const void* w, int w_dtype, int64_t ldw, const float* grad,

@@ -781,3 +781,47 @@ def test_prepare_subgroup_gathers_exact(R_s, C, wdt, ldpad, perm_on):
     exp_q = (scale.cpu().unsqueeze(1) * cf[:, invperm.cpu()]).to(torch.float16)
     torch.testing.assert_close(q.cpu(), exp_q, rtol=0, atol=0, equal_nan=True)
     assert int(flag.item()) == 1
+
+
+@pytest.mark.parametrize("sym", [True, False])
+@pytest.mark.parametrize("n,gs", [(1, -1), (63, -1), (65, -1), (257, -1), (300, 100), (1024, -1), (1025, -1),
+                                  (2050, 1030), (16384, -1), (16385, -1)])
+def test_find_params_mse_widths(n, gs, sym):
+    """The clip search around its edges: partial waves and batches of candidates, a wave or a
+    workgroup per (row, group), rows staged in LDS or read in place; an all-zero row, one-sign
+    rows, a row of subnormals (IEEE divide and powf), a row with NaN and one with infinity.
+    A choice other than the oracle's must have an error sum within 2^-13 of the oracle's: both sum
+    n <= 16385 non-negative terms in 32 bits, each order within 2 (n / 256 + 12) 2^-24 < 2^-16,
+    and a power within 2^-23, over a factor of 4."""
+    R = 9 if n > 4096 else 24
+    r = rng(1000 + n + sym)
+    W = torch.from_numpy(r.standard_normal((R, n)).astype(np.float32) * 0.03)
+    W[1] = 0
+    W[2] = W[2].abs()
+    W[3] = -W[3].abs()
+    W[4] = W[4] * 1e-38
+    W[5, n // 2] = float("nan")
+    W[6, n // 3] = float("inf")
+    q = make_quantizer(4, sym, mse=True)
+    scale, zero = K.find_params_mse(W.to(DEV), int(q.maxq), sym, group_size=gs)
+    width = gs if gs > 0 else n
+    maxq = float(q.maxq)
+
+    def clip_err(x, s_, z_):
+        x, s_, z_ = x.double(), float(s_), float(z_)
+        if sym:
+            qv = s_ * torch.clamp(torch.round(x / s_), -(maxq + 1), maxq)
+        else:
+            qv = s_ * (torch.clamp(torch.round(x / s_) + z_, 0, maxq) - z_)
+        return float(((qv - x).abs() ** 2.4).sum())
+
+    for k, c0 in enumerate(range(0, n, width)):
+        Wg = W[:, c0:c0 + width]
+        qo = make_quantizer(4, sym, mse=True)
+        qo.find_params(Wg.clone())
+        so, zo = qo.scale.flatten(), qo.zero.flatten()
+        sg, zg = scale[k].cpu(), zero[k].cpu()
+        same = ((sg == so) | (sg.isnan() & so.isnan())) & ((zg == zo) | (zg.isnan() & zo.isnan()))
+        for i in torch.nonzero(~same).flatten().tolist():
+            e_gpu, e_ora = clip_err(Wg[i], sg[i], zg[i]), clip_err(Wg[i], so[i], zo[i])
+            assert abs(e_gpu - e_ora) <= 2.0 ** -13 * e_ora, (i, e_gpu, e_ora)
