@@ -394,7 +394,8 @@ def unpack_dequant(packed, C, nbits, scales=None, g_idx=None, q_dtype=torch.floa
             g_idx = _cin(g_idx, "g_idx", torch.int32)
             if g_idx.numel() != C:
                 raise ValueError("unpack_dequant: g_idx must be int32 [C]")
-            if int(g_idx.min()) < 0 or int(g_idx.max()) >= scales.shape[0]:
+            lo, hi = torch.stack(torch.aminmax(g_idx)).tolist()     # one read-back
+            if lo < 0 or hi >= scales.shape[0]:
                 raise ValueError("unpack_dequant: g_idx out of range of the scale table")
         elif scales.shape[0] != 1:
             raise ValueError("unpack_dequant: several scale groups need g_idx")

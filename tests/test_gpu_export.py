@@ -103,3 +103,33 @@ def test_export_after_free_fails_loudly():
     g.free()
     with pytest.raises(RuntimeError):
         export_packed(g)
+
+
+@pytest.mark.parametrize("nbits", [2, 5, 7, 9, 13, 16])
+@pytest.mark.parametrize("R,C,off", [(1, 8, 0), (3, 7, 0), (2050, 40, 0), (9000, 24, 0), (5, 264, 1), (2, 32768, 0),
+                                     (2, 32776, 0), (3, 4097, 3)])
+def test_pack_unpack_edges(nbits, R, C, off):
+    """Packing by staged rows (1 to 8 rows a workgroup, rows at and past the LDS limit, unaligned rows
+    read from a wider buffer) and unpacking 8 columns a thread (a ragged last unit, mixed scale
+    groups, unaligned outputs) against the format's CPU definition, exactly."""
+    r = rng(nbits * 1000 + C)
+    half = 1 << (nbits - 1)
+    codes = r.integers(-half, half, size=(R, C)).astype(np.int16)
+    want = pack_rows(codes, nbits)
+    perm = torch.from_numpy(r.permutation(C))
+    wide = torch.zeros((R, C + 8), dtype=torch.int16)
+    wide[:, off:off + C] = torch.from_numpy(codes)[:, perm]
+    src = wide.to(DEV)[:, off:off + C]                       # row stride C + 8, base offset `off`
+    got = K.pack_codes(src, nbits, invperm=torch.argsort(perm).to(DEV))
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want)
+    ng = 3
+    scales = torch.from_numpy(r.lognormal(size=(ng, R)).astype(np.float32))
+    g_idx = torch.from_numpy(r.integers(0, ng, size=C).astype(np.int32))
+    g_idx[:min(C, 16)] = 1                                   # a unit of one group
+    for dt in (torch.float16, torch.float32):
+        q, back = K.unpack_dequant(got, C, nbits, scales.to(DEV), g_idx.to(DEV), dt, want_codes=True)
+        assert np.array_equal(back.cpu().numpy(), codes)
+        exp = (scales[g_idx.long()].T * torch.from_numpy(codes).float()).to(dt)
+        assert torch.equal(q.cpu(), exp)
+    with pytest.raises(ValueError):
+        K.unpack_dequant(got, C, nbits, scales.to(DEV), torch.full((C,), ng, dtype=torch.int32, device=DEV))
