@@ -526,6 +526,19 @@ __device__ __forceinline__ void split_staged(const uint8_t* st, int wave, int la
              *reinterpret_cast<const float4*>(sp + 16), sc, p);
 }
 
+// A wave's 32 x 32 blocks: of an off-diagonal tile the 8 row blocks of its column block; of a
+// diagonal tile, whose 36 blocks of the upper triangle are to be computed, 5 (column blocks 0-3)
+// or 4 (4-7): row blocks c, c + 1, .. around the tile.  Every pair of row and column blocks is
+// then taken once, as block (r, c) or, below the diagonal, as the transpose of (c, r), and each
+// wave has 4 or 5 blocks.  (With the upper blocks of its own columns, 1 to 8 a wave, the SIMDs had
+// equal work too, but the wave with 8 set the step's time alone: 0.71 -> 0.55 us a step in fp16,
+// 0.80 -> 0.65 in bf16, one tile on the GPU; an off-diagonal step takes 0.77 and 0.93.)
+template <bool DIAG>
+constexpr int XBLK = DIAG ? 5 : 8;
+__host__ __device__ constexpr int diag_lim(int cbw) { return cbw < 4 ? 5 : 4; }
+template <bool DIAG>
+__device__ __forceinline__ int diag_rows(int cbw, int b) { return DIAG ? (cbw + b) & 7 : b; }
+
 // One 16-token step k of a wave.  KP = (k - kbeg) % 2 selects the register buffers (row
 // fragments a and pieces p of step k, both read or made during step k-1); CUR, NXT, FILL are
 // the stages of steps k, k+1 and k+XDEPTH-1.  Every wave's staging of steps k and k+1 was
@@ -549,13 +562,14 @@ __device__ __forceinline__ void split_staged(const uint8_t* st, int wave, int la
 // staging (wave 0, lanes 0-3, a branch) comes last, so the step's main work is one scheduling
 // region.  Its vmcnt accounting is unchanged: wave 0's saliency load of step k+XDEPTH-1 still
 // follows that step's row / column loads.
-// DIAG (a diagonal tile): row blocks below this wave's column block hold only the discarded
-// lower triangle, so their row fragments are not read and their MFMAs not issued (bi < lim).
+// DIAG (a diagonal tile): the wave's blocks are `lim` row blocks from its own column block on,
+// around the tile (see diag_rows), in pairs of which the last may be half; the next step's four
+// token pairs are split in the first two.
 template <typename TX, int PC, bool DIAG, int KP, int CUR, int NXT, int FILL>
-__device__ __forceinline__ void split_step(uint4 (&p)[2][PC], uint4 (&a)[2][8], floatx16 (&acc)[8],
+__device__ __forceinline__ void split_step(uint4 (&p)[2][PC], uint4 (&a)[2][XBLK<DIAG>], floatx16 (&acc)[XBLK<DIAG>],
                                            const XStages& L, const uint16_t* pa, const uint16_t* pb,
                                            const float* sg, float sc, int wave, int lane, int64_t k,
-                                           int64_t last, int lim) {
+                                           int64_t last, int cbw, int lim) {
   typedef XType<TX> T;
   typedef typename T::v8 v8;
   constexpr int NP = 1 - KP;
@@ -579,23 +593,30 @@ __device__ __forceinline__ void split_step(uint4 (&p)[2][PC], uint4 (&a)[2][8], 
   const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
   const uint32_t xw[4] = {b.x, b.y, b.z, b.w};
   uint32_t o[XNPMAX][4];
+  auto split = [&](int j) __attribute__((always_inline)) {
+    split_pair<TX, PC>(xw[j], sv[2 * j], sv[2 * j + 1], sc, o[0][j], o[1][j], o[2][j]);
+  };
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < (XBLK<DIAG> + 1) / 2; ++j) {
     const int b0 = 2 * j, b1 = 2 * j + 1;
+    if (DIAG && b0 >= lim) break;
 #pragma unroll
     for (int q = PC - 1; q >= 0; --q) {
-      if (!DIAG || b0 < lim)
-        acc[b0] = T::mfma(__builtin_bit_cast(v8, a[KP][b0]), __builtin_bit_cast(v8, p[KP][q]), acc[b0]);
-      if (!DIAG || b1 < lim)
+      acc[b0] = T::mfma(__builtin_bit_cast(v8, a[KP][b0]), __builtin_bit_cast(v8, p[KP][q]), acc[b0]);
+      if (b1 < XBLK<DIAG>)
         acc[b1] = T::mfma(__builtin_bit_cast(v8, a[KP][b1]), __builtin_bit_cast(v8, p[KP][q]), acc[b1]);
       __builtin_amdgcn_sched_barrier(0);
       if (q == PC - 1) {            // after the first MFMA pair: the pair's next-step row fragments
-        if (!DIAG || b0 < lim) a[NP][b0] = *reinterpret_cast<const uint4*>(nxt + b0 * 1024);
-        if (!DIAG || b1 < lim) a[NP][b1] = *reinterpret_cast<const uint4*>(nxt + b1 * 1024);
+        a[NP][b0] = *reinterpret_cast<const uint4*>(nxt + diag_rows<DIAG>(cbw, b0) * 1024);
+        if (b1 < XBLK<DIAG>) a[NP][b1] = *reinterpret_cast<const uint4*>(nxt + diag_rows<DIAG>(cbw, b1) * 1024);
       }
-      if (q == PC - 2)              // after the second: the split of token pair j
-        split_pair<TX, PC>(xw[j], sv[2 * j], sv[2 * j + 1], sc, o[0][j], o[1][j], o[2][j]);
+      if (!DIAG) {
+        if (q == PC - 2) split(j);              // after the second: the split of token pair j
+      } else if (j < 2) {
+        if (q == PC - 2) split(2 * j);          // (two to a pair)
+        if (q == 0) split(2 * j + 1);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -607,12 +628,13 @@ __device__ __forceinline__ void split_step(uint4 (&p)[2][PC], uint4 (&a)[2][8], 
 // Steps k .. k+nsteps-1 (nsteps <= XDEPTH) of the unrolled schedule: step k+J uses stage J,
 // reads stage J+1 and refills stage J-1 (mod XDEPTH), and register buffer J % 2.
 template <typename TX, int PC, bool DIAG, int... J>
-__device__ __forceinline__ void split_round(uint4 (&p)[2][PC], uint4 (&a)[2][8], floatx16 (&acc)[8],
+__device__ __forceinline__ void split_round(uint4 (&p)[2][PC], uint4 (&a)[2][XBLK<DIAG>],
+                                            floatx16 (&acc)[XBLK<DIAG>],
                                             const XStages& L, const uint16_t* pa, const uint16_t* pb,
                                             const float* sg, float sc, int wave, int lane, int64_t k,
-                                            int64_t last, int lim, int nsteps, std::integer_sequence<int, J...>) {
+                                            int64_t last, int cbw, int lim, int nsteps, std::integer_sequence<int, J...>) {
   ((J < nsteps ? split_step<TX, PC, DIAG, J % 2, J, (J + 1) % XDEPTH, (J + XDEPTH - 1) % XDEPTH>(
-                     p, a, acc, L, pa, pb, sg, sc, wave, lane, k + J, last, lim)
+                     p, a, acc, L, pa, pb, sg, sc, wave, lane, k + J, last, cbw, lim)
                : void()),
    ...);
 }
@@ -636,7 +658,7 @@ __device__ __forceinline__ void split_tile(const uint16_t* __restrict__ XB, int6
   const int fr = lane & 31, fh = lane >> 5;
   const int cbw = split_colblock(wave);
   const int Cw = C0 + 32 * cbw;
-  const int lim = DIAG ? cbw + 1 : 8;   // row blocks this wave computes
+  const int lim = DIAG ? diag_lim(cbw) : 8;   // row blocks this wave computes
   const int ncb = (C + 31) / 32;
 
   // Fragment sources in the fragment-blocked chunk: block cb of 32 columns, step k at
@@ -646,9 +668,10 @@ __device__ __forceinline__ void split_tile(const uint16_t* __restrict__ XB, int6
   const uint16_t* pb = XB + ((int64_t)min(Cw / 32, ncb - 1) * nks * 64 + lane) * 8;
   const float sc = scl[min(Cw + fr, C - 1)];
 
-  floatx16 acc[8];
+  constexpr int NB = XBLK<DIAG>;
+  floatx16 acc[NB];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
 
@@ -657,15 +680,14 @@ __device__ __forceinline__ void split_tile(const uint16_t* __restrict__ XB, int6
   const int64_t last = kend - 1;
 #pragma unroll
   for (int h = 0; h < XDEPTH - 1; ++h) stage_step(L.s[h], pa, pb, sg, wave, lane, min(kbeg + h, last));
-  uint4 p[2][PC], a[2][8];
+  uint4 p[2][PC], a[2][NB];
   XWAIT_VM(2 * (XDEPTH - 2));         // this wave's staging of step kbeg
   RQ_STAGE_BARRIER();       // and the other waves'
   split_staged<TX, PC>(L.s[0], wave, lane, sc, p[0]);
   {
     const uint8_t* cur = static_cast<const uint8_t*>(__builtin_assume_aligned(L.s[0] + lane * 16, 16));
 #pragma unroll
-    for (int bi = 0; bi < 8; ++bi)
-      if (!DIAG || bi < lim) a[0][bi] = *reinterpret_cast<const uint4*>(cur + bi * 1024);
+    for (int bi = 0; bi < NB; ++bi) a[0][bi] = *reinterpret_cast<const uint4*>(cur + diag_rows<DIAG>(cbw, bi) * 1024);
   }
 
   const int64_t n = kend - kbeg;
@@ -673,97 +695,225 @@ __device__ __forceinline__ void split_tile(const uint16_t* __restrict__ XB, int6
   static_assert(XDEPTH % 2 == 0, "register buffers alternate by step");
   constexpr auto round = std::make_integer_sequence<int, XDEPTH>();
   for (; k + XDEPTH <= kend; k += XDEPTH)
-    split_round<TX, PC, DIAG>(p, a, acc, L, pa, pb, sg, sc, wave, lane, k, last, lim, XDEPTH, round);
-  split_round<TX, PC, DIAG>(p, a, acc, L, pa, pb, sg, sc, wave, lane, k, last, lim, (int)(n % XDEPTH), round);
+    split_round<TX, PC, DIAG>(p, a, acc, L, pa, pb, sg, sc, wave, lane, k, last, cbw, lim, XDEPTH, round);
+  split_round<TX, PC, DIAG>(p, a, acc, L, pa, pb, sg, sc, wave, lane, k, last, cbw, lim, (int)(n % XDEPTH),
+                            round);
   XWAIT_VM(0);                        // no staging left in flight when the workgroup moves on
 
   if (part) {
-    // token slice: hand the (still scaled) partial tile to the workspace (zeros for the row
-    // blocks a diagonal tile does not compute)
+    // segment of an item: hand the (still scaled) partial tile to the workspace
 #pragma unroll
-    for (int bi = 0; bi < 8; ++bi)
+    for (int bi = 0; bi < NB; ++bi)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) part[(bi * 16 + e) * XTHREADS + tid] = (DIAG && bi >= lim) ? 0.0f : acc[bi][e];
+      for (int e = 0; e < 16; ++e)
+        if (!DIAG || bi < lim) part[(bi * 16 + e) * XTHREADS + tid] = acc[bi][e];
     return;
   }
-  // H[g][i][j] += acc * 2^-e_j   (32x32 block layout: i = 8*(e/4) + 4*(lane/32) + e%4, j = lane%32)
-  // The 16 loads of a block are issued together, then the 16 stores.
+  // H[g][i][j] += acc * 2^-e_j   (32x32 block layout: i = 8*(e/4) + 4*(lane/32) + e%4, j = lane%32;
+  // a diagonal tile's blocks below its diagonal go to H[g][j][i])
+  // The 16 loads of a block are issued together, before the 16 stores of the block before it.
   const int j = Cw + fr;
   const float inv = (j < C) ? 1.0f / scl[j] : 0.0f;
+  if constexpr (!DIAG) {
+    float hv[2][16];
+    auto load = [&](int bi, float (&h)[16]) {
 #pragma unroll
-  for (int bi = 0; bi < 8; ++bi) {
-    if (DIAG && bi >= lim) continue;   // below the diagonal: nothing was accumulated
-    float hv[16];
+      for (int e = 0; e < 16; ++e) {
+        const int i = R0 + 32 * bi + 8 * (e >> 2) + 4 * fh + (e & 3);
+        h[e] = (i < C && j < C) ? Hg[(int64_t)i * C + j] : 0.0f;
+      }
+    };
+    load(0, hv[0]);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int i = R0 + 32 * bi + 8 * (e >> 2) + 4 * fh + (e & 3);
-      hv[e] = (i < C && j < C) ? Hg[(int64_t)i * C + j] : 0.0f;
+    for (int bi = 0; bi < 8; ++bi) {
+      if (bi + 1 < 8) load(bi + 1, hv[(bi + 1) & 1]);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int i = R0 + 32 * bi + 8 * (e >> 2) + 4 * fh + (e & 3);
+        if (i < C && j < C) Hg[(int64_t)i * C + j] = hv[bi & 1][e] + acc[bi][e] * inv;
+      }
     }
+  } else {
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int i = R0 + 32 * bi + 8 * (e >> 2) + 4 * fh + (e & 3);
-      if (i < C && j < C) Hg[(int64_t)i * C + j] = hv[e] + acc[bi][e] * inv;
+    for (int bi = 0; bi < NB; ++bi) {
+      if (bi >= lim) continue;
+      const int rb = diag_rows<DIAG>(cbw, bi);
+      const int i0 = R0 + 32 * rb + 4 * fh;
+      // element (i, j), or (j, i) below the diagonal
+      float* ph = Hg + (rb > cbw ? (int64_t)j * C + i0 : (int64_t)i0 * C + j);
+      const int64_t st = rb > cbw ? 1 : C;
+      float hv[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int d = 8 * (e >> 2) + (e & 3);
+        hv[e] = (i0 + d < C && j < C) ? ph[d * st] : 0.0f;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int d = 8 * (e >> 2) + (e & 3);
+        if (i0 + d < C && j < C) ph[d * st] = hv[e] + acc[bi][e] * inv;
+      }
     }
   }
 }
 
-// The last slice of a split item adds the S partials (in slice order) to H.
-__device__ __forceinline__ void reduce_split_slices(const float* __restrict__ part0, int S,
-                                                    float* __restrict__ Hg, const float* __restrict__ scl,
-                                                    int R0, int C0, int C, const float* __restrict__ rsc = nullptr) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int fr = lane & 31, fh = lane >> 5;
-  const int j = C0 + 32 * split_colblock(wave) + fr;   // the column the slices' thread held
-  const float inv = (j < C) ? 1.0f / scl[j] : 0.0f;
-  // per accumulator block: the S partials of its 16 outputs loaded 8 slices at a time (S
-  // uniform), added in slice order
-#pragma unroll 1
-  for (int bi = 0; bi < 8; ++bi) {
-    float sums[16];
-#pragma unroll 1
-    for (int q0 = 0; q0 < S; q0 += 8) {
-      float v[16][8];
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-          v[e][q] = (q0 + q < S) ? __hip_atomic_load(part0 + (int64_t)(q0 + q) * XPART + (bi * 16 + e) * XTHREADS + tid,
-                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                 : 0.0f;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        float acc = q0 == 0 ? v[e][0] : sums[e] + v[e][0];
-#pragma unroll
-        for (int q = 1; q < 8; ++q)
-          if (q0 + q < S) acc += v[e][q];
-        sums[e] = acc;
-      }
+// The tail of a launch (the item list's last items, from `full` on): `od` off-diagonal items, then
+// `dg` diagonal ones.  The off-diagonal items' steps, laid end to end, are cut into `nod` equal
+// ranges, one per workgroup: a range ends inside one item and the next begins there.  Each
+// diagonal item is cut into `sd` equal slices.  The part of an item in a range (or slice) is a
+// segment; one that is not the whole item leaves a partial tile in the workspace, and
+// k_split_reduce adds them to H in token order.  nod = od, sd = 1: every item whole.
+struct TailPlan {
+  int od, dg, nod, sd;
+  __host__ __device__ int items() const { return od + dg; }
+  __host__ __device__ int wgs() const { return nod + dg * sd; }
+  // partial tiles: off-diagonal ranges have at most two, slot 2 w for the segment of range w that
+  // starts inside an item and 2 w + 1 for one that starts it; then the diagonal slices
+  __host__ __device__ int od_slots() const { return nod > od ? 2 * nod : 0; }
+  __host__ __device__ int slots() const { return od_slots() + (sd > 1 ? dg * sd : 0); }
+  __host__ __device__ __forceinline__ int64_t cut(int w, int64_t nks) const { return nks * od * w / nod; }
+  // Segment s of workgroup w: its item, steps and slot; false when it has none.
+  __host__ __device__ __forceinline__ bool segment(int w, int s, int64_t nks, int& item, int64_t& kb, int64_t& ke,
+                                                   int64_t& slot) const {
+    if (w >= nod) {
+      const int d = w - nod, q = d % sd;
+      item = od + d / sd;
+      kb = nks * q / sd;
+      ke = nks * (q + 1) / sd;
+      slot = od_slots() + d;
+      return s == 0;
     }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float sum = sums[e];
-      const int i = R0 + 32 * bi + 8 * (e >> 2) + 4 * fh + (e & 3);
-      if (i < C && j < C) {
-        float* ph = Hg + (int64_t)i * C + j;
-        if (rsc)   // fp32 X: 2^-(ex_i + e_j), applied in fp64 (exact)
-          *ph = *ph + (float)((double)sum * ((double)inv / (double)rsc[i]));
-        else
-          *ph = *ph + sum * inv;
-      }
-    }
+    const int64_t u = cut(w, nks), z = cut(w + 1, nks);
+    item = (int)(u / nks) + s;
+    const int64_t a = nks * item;
+    kb = u > a ? u - a : 0;
+    ke = z < a + nks ? z - a : nks;
+    slot = 2 * (int64_t)w + (kb == 0 ? 1 : 0);
+    return kb < ke;
   }
+};
+
+// Position of block b when n blocks are dealt to the 8 XCDs (block b runs on XCD b % 8 up to a
+// rotation) as contiguous runs.
+__device__ __forceinline__ int xcd_run(int b, int n) {
+  const int x = b % 8;
+  return x * (n / 8) + min(x, n % 8) + b / 8;
+}
+
+// H += the partial tiles of the tail's items, added in token order.  HBM-bound: 256 KB per segment
+// and twice that for the tile.  It was the last slice's work before (one workgroup per item, behind
+// an agent-scope fence in every slice); a launch of its own spreads an item over 16 workgroups of
+// 8 accumulator rows.  63 items of 4 slices (C = 1365, G = 3, 2505 tokens): 223 -> 62 + 14 us for
+// the call's product kernels.
+// rsc: fp32 X, the row exponents 2^-ex_i (applied in fp64, exact).
+// circ: a diagonal tile's blocks are numbered as diag_rows does (else block bi is row block bi).
+__global__ __launch_bounds__(XTHREADS) void k_split_reduce(const float* __restrict__ ws, TailPlan P, int64_t nks,
+                                                           int full, int ntarg, int nt, int C, int circ,
+                                                           const float* __restrict__ scale,
+                                                           const float* __restrict__ rsc, HTargets tg) {
+  const int it = blockIdx.x;
+  const bool od = it < P.od;
+  if (od ? P.nod <= P.od : P.sd == 1) return;     // the kind's items ran whole
+  int g, ti, tj;
+  item_tile(full + it, ntarg, nt, g, ti, tj);
+  const int R0 = ti * XT, C0 = tj * XT;
+  const int bi = blockIdx.y >> 1, e0 = 8 * (blockIdx.y & 1);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int cbw = split_colblock(__builtin_amdgcn_readfirstlane(tid >> 6));
+  const bool diag = ti == tj;
+  if (diag && (circ ? bi >= diag_lim(cbw) : bi > cbw)) return;      // not one of the wave's blocks
+  const int rb = diag && circ ? (cbw + bi) & 7 : bi;
+  const bool flip = rb > cbw && diag;             // below the diagonal: the transpose
+  int w0, w1;                                     // the workgroups of the item's segments
+  if (od) {
+    w0 = (int)(nks * it * P.nod / (nks * P.od));
+    while (P.cut(w0 + 1, nks) <= nks * it) ++w0;  // (cut() rounds down)
+    w1 = w0;
+    while (P.cut(w1 + 1, nks) < nks * (it + 1)) ++w1;
+  } else {
+    w0 = P.nod + (it - P.od) * P.sd;
+    w1 = w0 + P.sd - 1;
+  }
+  const int fr = lane & 31, fh = lane >> 5;
+  const int j = C0 + 32 * cbw + fr;               // the column the segments' thread held
+  float* Hg = tg.H[g];
+  const int64_t off = (int64_t)(bi * 16 + e0) * XTHREADS + tid;
+  auto addr = [&](int e) -> float* {
+    const int i = R0 + 32 * rb + 8 * ((e0 + e) >> 2) + 4 * fh + (e & 3);
+    if (i >= C || j >= C) return nullptr;
+    return Hg + (flip ? (int64_t)j * C + i : (int64_t)i * C + j);
+  };
+  float hv[8], sum[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float* q = addr(e);
+    hv[e] = q ? *q : 0.0f;
+    sum[e] = 0.0f;
+  }
+  bool any = false;
+  for (int w = w0; w <= w1; ++w) {
+    int item;
+    int64_t kb, ke, slot;
+    bool has = P.segment(w, 0, nks, item, kb, ke, slot);
+    if (od && item < it) has = P.segment(w, it - item, nks, item, kb, ke, slot);
+    if (!has) continue;
+    if (ke - kb == nks) return;                   // the whole item: already in H
+    const float* part = ws + slot * XPART + off;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float v = part[e * XTHREADS];
+      sum[e] = any ? sum[e] + v : v;
+    }
+    any = true;
+  }
+  const float inv = (j < C) ? 1.0f / scale[(int64_t)g * C + j] : 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int i = R0 + 32 * rb + 8 * ((e0 + e) >> 2) + 4 * fh + (e & 3);
+    float* q = addr(e);
+    if (q) *q = hv[e] + (rsc ? (float)((double)sum[e] * ((double)inv / (double)rsc[i])) : sum[e] * inv);
+  }
+}
+
+// A wave-uniform 64-bit value, in scalar registers.
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// A workgroup's work: the whole item `logical`, or (w >= 0) the segments of the tail's workgroup
+// w.  One call site of `tile` for both, so its body is compiled once.
+template <typename F>
+__device__ __forceinline__ void whole_or_tail(F&& tile, int logical, int w, const TailPlan& P, int64_t nks, int full,
+                                              int total, float* __restrict__ ws) {
+  int s = 0;
+  bool more;
+  do {
+    int64_t kb = 0, ke = nks, slot = 0;
+    int item = logical;
+    more = false;
+    if (w >= 0) {
+      more = P.segment(w, s++, nks, item, kb, ke, slot) && w < P.nod;
+      item += full;
+    }
+    kb = uniform64(kb);
+    ke = uniform64(ke);
+    item = __builtin_amdgcn_readfirstlane(item);
+    if (kb < ke && item < total) tile(item, kb, ke, ke - kb == nks ? nullptr : ws + slot * XPART);
+    __syncthreads();                              // the staging ring is free for the next segment
+    more = __builtin_amdgcn_readfirstlane((int)more) != 0;
+  } while (more);
 }
 
 // One launch covers a segment of the item list: its `segn` whole items from list position seg0
 // on (od_seg of them off-diagonal), dealt to the XCDs as item_position describes, followed in the
-// last segment by the tail's token slices (the list's items from `full` on, S slices each).
+// last segment by the tail's token slices (the list's items from `full` on).
 template <typename TX, int PC>
 __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split(
     const uint16_t* __restrict__ XB, int C, const float* __restrict__ sT, int64_t lds_stride,
     const float* __restrict__ scale, HTargets tg, int ntarg, int nt, int ntiles, int64_t nks, int seg0,
-    int segn, int od_seg, int full, int S, float* __restrict__ ws, int* __restrict__ cnt) {
+    int segn, int od_seg, int full, TailPlan P, float* __restrict__ ws) {
   __shared__ __attribute__((aligned(16))) uint8_t lds0[XSTAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds1[XSTAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds2[XSTAGE];
@@ -772,49 +922,25 @@ __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split(
   __shared__ __attribute__((aligned(16))) uint8_t lds5[XSTAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds6[XSTAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds7[XSTAGE];
-  __shared__ int last_slice;
   static_assert(XDEPTH == 8, "stage arrays");
   const XStages L{{lds0, lds1, lds2, lds3, lds4, lds5, lds6, lds7}};
   // Same schedule as k_hessian_accum: XCD-aware order for whole items, then the token
   // slices of the tail items.
   const int total = ntiles * ntarg;
   const int b = blockIdx.x;
-  int logical, slice = -1;
-  int64_t kbeg = 0, kend = nks;
-  if (b < segn) {
-    logical = seg0 + item_position(b, segn, od_seg);
-  } else {
-    const int tb = b - segn;
-    logical = full + tb / S;
-    slice = tb % S;
-    kbeg = nks * slice / S;
-    kend = nks * (slice + 1) / S;
-  }
-  if (logical >= total) return;
-  int g, ti, tj;
-  item_tile(logical, ntarg, nt, g, ti, tj);
-  const int R0 = ti * XT, C0 = tj * XT;
-  float* Hg = tg.H[g];
-  const float* scl = scale + (int64_t)g * C;
-  float* part0 = (slice >= 0) ? ws + (int64_t)(logical - full) * S * XPART : nullptr;
-  float* part = part0 ? part0 + (int64_t)slice * XPART : nullptr;
-  if (R0 == C0)
-    split_tile<TX, PC, true>(XB, nks, C, sT + (int64_t)g * lds_stride, scl, Hg, R0, C0, kbeg, kend, part, L);
-  else
-    split_tile<TX, PC, false>(XB, nks, C, sT + (int64_t)g * lds_stride, scl, Hg, R0, C0, kbeg, kend, part, L);
-  if (!part) return;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int* cp = cnt + (logical - full);
-    const int prev = atomicAdd(cp, 1);
-    last_slice = (prev == S - 1);
-    if (last_slice) atomicExch(cp, 0);
-  }
-  __syncthreads();
-  if (!last_slice) return;
-  __threadfence();
-  reduce_split_slices(part0, S, Hg, scl, R0, C0, C);
+  auto tile = [&](int logical, int64_t kbeg, int64_t kend, float* part) __attribute__((always_inline)) {
+    int g, ti, tj;
+    item_tile(logical, ntarg, nt, g, ti, tj);
+    const int R0 = ti * XT, C0 = tj * XT;
+    float* Hg = tg.H[g];
+    const float* scl = scale + (int64_t)g * C;
+    if (R0 == C0)
+      split_tile<TX, PC, true>(XB, nks, C, sT + (int64_t)g * lds_stride, scl, Hg, R0, C0, kbeg, kend, part, L);
+    else
+      split_tile<TX, PC, false>(XB, nks, C, sT + (int64_t)g * lds_stride, scl, Hg, R0, C0, kbeg, kend, part, L);
+  };
+  const int w = b < segn ? -1 : xcd_run(b - segn, P.wgs());
+  whole_or_tail(tile, b < segn ? seg0 + item_position(b, segn, od_seg) : 0, w, P, nks, full, total, ws);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -990,7 +1116,8 @@ __device__ __forceinline__ void split_tile32(const uint16_t* __restrict__ XH, co
 #pragma unroll
     for (int bi = 0; bi < 8; ++bi)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) part[(bi * 16 + e) * XTHREADS + tid] = (DIAG && bi >= lim) ? 0.0f : acc[bi][e];
+      for (int e = 0; e < 16; ++e)
+        if (!DIAG || bi < lim) part[(bi * 16 + e) * XTHREADS + tid] = acc[bi][e];
     return;
   }
   // H[g][i][j] += acc * 2^-(ex_i + e_j), the two exact scalings applied in fp64
@@ -1016,55 +1143,31 @@ __device__ __forceinline__ void split_tile32(const uint16_t* __restrict__ XH, co
 __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split32(
     const uint16_t* __restrict__ XH, const uint16_t* __restrict__ XL, const float* __restrict__ XC, int C,
     const float* __restrict__ sT, int64_t lds_stride, const float* __restrict__ scale,
-    const float* __restrict__ rscale, HTargets tg, int ntarg, int nt, int ntiles, int64_t nks, int full, int S,
-    float* __restrict__ ws, int* __restrict__ cnt) {
+    const float* __restrict__ rscale, HTargets tg, int ntarg, int nt, int ntiles, int64_t nks, int full,
+    TailPlan P, float* __restrict__ ws) {
   __shared__ __attribute__((aligned(16))) uint8_t lds0[X3_STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds1[X3_STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds2[X3_STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t lds3[X3_STAGE];
-  __shared__ int last_slice;
   static_assert(X32DEPTH == 4, "stage arrays");
   const XStages L{{lds0, lds1, lds2, lds3}};
   const int total = ntiles * ntarg;
   const int b = blockIdx.x;
-  int logical, slice = -1;
-  int64_t kbeg = 0, kend = nks;
-  if (b < full) {
-    logical = item_position(b, full, nt * (nt - 1) / 2 * ntarg);
-  } else {
-    const int tb = b - full;
-    logical = full + tb / S;
-    slice = tb % S;
-    kbeg = nks * slice / S;
-    kend = nks * (slice + 1) / S;
-  }
-  if (logical >= total) return;
-  int g, ti, tj;
-  item_tile(logical, ntarg, nt, g, ti, tj);
-  const int R0 = ti * XT, C0 = tj * XT;
-  float* Hg = tg.H[g];
-  const float* scl = scale + (int64_t)g * C;
-  float* part0 = (slice >= 0) ? ws + (int64_t)(logical - full) * S * XPART : nullptr;
-  float* part = part0 ? part0 + (int64_t)slice * XPART : nullptr;
-  if (R0 == C0)
-    split_tile32<true>(XH, XL, XC, nks, C, sT + (int64_t)g * lds_stride, scl, rscale, Hg, R0, C0, kbeg, kend,
-                       part, L);
-  else
-    split_tile32<false>(XH, XL, XC, nks, C, sT + (int64_t)g * lds_stride, scl, rscale, Hg, R0, C0, kbeg, kend,
-                        part, L);
-  if (!part) return;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int* cp = cnt + (logical - full);
-    const int prev = atomicAdd(cp, 1);
-    last_slice = (prev == S - 1);
-    if (last_slice) atomicExch(cp, 0);
-  }
-  __syncthreads();
-  if (!last_slice) return;
-  __threadfence();
-  reduce_split_slices(part0, S, Hg, scl, R0, C0, C, rscale);
+  auto tile = [&](int logical, int64_t kbeg, int64_t kend, float* part) __attribute__((always_inline)) {
+    int g, ti, tj;
+    item_tile(logical, ntarg, nt, g, ti, tj);
+    const int R0 = ti * XT, C0 = tj * XT;
+    float* Hg = tg.H[g];
+    const float* scl = scale + (int64_t)g * C;
+    if (R0 == C0)
+      split_tile32<true>(XH, XL, XC, nks, C, sT + (int64_t)g * lds_stride, scl, rscale, Hg, R0, C0, kbeg, kend, part,
+                         L);
+    else
+      split_tile32<false>(XH, XL, XC, nks, C, sT + (int64_t)g * lds_stride, scl, rscale, Hg, R0, C0, kbeg, kend, part,
+                          L);
+  };
+  const int w = b < full ? -1 : xcd_run(b - full, P.wgs());
+  whole_or_tail(tile, b < full ? item_position(b, full, nt * (nt - 1) / 2 * ntarg) : 0, w, P, nks, full, total, ws);
 }
 
 // Pre-pass over one 64-column x 256-token block of X: the block in the fragment-blocked
@@ -1669,10 +1772,7 @@ int split_slots() { return kernel_slots(k_hessian_split<__half, 3>, XTHREADS, 1)
 // Items of the last, partly filled round and their slice count: the most slices that still
 // fit the tail into one round (S = slots / tail, S <= maxS, at least 4 token slabs per slice).
 // Measured at C = 4096 (tails of 32, 64, 96 and 136 items on 256 slots: best S = 6-8, 3-4, 2 and
-// 1-3) and 14336 (240 items: 1).  Splitting further, into more rounds, loses: besides each
-// slice's partial tile and the last slice's reduction, the power-limited clock rises when fewer
-// CUs are busy, so a tail on part of the GPU costs less than its idle share.  The split kernels
-// reduce up to 16 slices, the fp32 kernel up to 8.
+// 1-3) and 14336 (240 items: 1).  (The fp32 MFMA kernel; split_tail plans the split kernels'.)
 void tail_split(int64_t total, int64_t nslab, int slots, int maxS, int* tail, int* S) {
   *tail = 0;
   *S = 1;
@@ -1782,16 +1882,54 @@ int launch_act_square(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int
   return launch_act_square_t(static_cast<const float*>(x), ntok, ldx, C, tg, ntarg, l2_main, ws_act, s);
 }
 
+// How a launch's tail is cut (TailPlan).  S is the most slices per item that fit the tail into one
+// round, at most 16 and at least 4 steps each.  The diagonal items run as S slices, the off-diagonal
+// ones as S slices too where S is the most there may be (small calls: the same sums for one module's
+// call and a call for several), else as equal ranges over the workgroups that the diagonal
+// slices leave, if that is estimated to end sooner than S slices: a range costs XTAIL_RANGE steps
+// besides its own (filling the ring twice, two partial tiles and their reduction).  (A diagonal
+// element's terms are thus added in the same order whatever the ranges: act_order of a single
+// target's diagonal does not depend on them.)  Measured at C = 4096, one bf16 target of 32768 tokens (120 off-diagonal and
+// 16 diagonal items on 256 workgroups), product kernels of a call: every item whole 2.09 ms,
+// ranges 1.61 ms; C = 2048, four fp16 targets (112 + 32 items): 1.62 -> 1.50 ms for the call.
+constexpr int64_t XTAIL_RANGE = 60;
+
+TailPlan split_tail(int64_t total, int64_t od_items, int64_t nks, int slots, int64_t max_parts) {
+  TailPlan P{0, 0, 0, 1};
+  if (slots <= 0 || total <= 0 || total % slots == 0) return P;
+  const int tail = (int)(total % slots);
+  const int64_t full = total - tail;
+  P.od = (int)(od_items > full ? od_items - full : 0);
+  P.dg = tail - P.od;
+  P.nod = P.od;
+  const int64_t most = nks / 4 < 16 ? nks / 4 : 16;
+  int64_t S = slots / tail;
+  if (S > most) S = most;
+  if (S < 1) S = 1;
+  P.sd = (int)S;
+  P.nod = (int)(P.od * S);
+  if (P.slots() > max_parts) {                    // no room: whole items only
+    P.sd = 1;
+    P.nod = P.od;
+    return P;
+  }
+  const TailPlan R{P.od, P.dg, (int)(slots - P.dg * S), P.sd};
+  if (P.od > 0 && (S < most || full > 0) && R.nod > P.nod && R.slots() <= max_parts &&
+      nks * P.od / R.nod + XTAIL_RANGE < nks / S)
+    return R;
+  return P;
+}
+
 struct SplitLayout {
   int64_t ntok_p, nchunk, off_part, off_xt, off_st, off_m, off_a, off_s, off_scale, bytes;
 };
 
-SplitLayout split_layout(int64_t ntok, int C, int ntarg, int64_t tail, int S) {
+SplitLayout split_layout(int64_t ntok, int C, int ntarg, int64_t parts) {
   SplitLayout L;
   L.ntok_p = ((ntok + XTOK - 1) / XTOK) * XTOK;
   L.nchunk = L.ntok_p / XTOK;
   L.off_part = act_off() + act_plan(ntok, C).bytes;
-  L.off_xt = L.off_part + align256(tail * S * (int64_t)XPART * 4);
+  L.off_xt = L.off_part + align256(parts * (int64_t)XPART * 4);
   L.off_st = L.off_xt + align256((int64_t)((C + 31) / 32) * 32 * L.ntok_p * 2);
   L.off_m = L.off_st + align256((int64_t)ntarg * L.ntok_p * 4);
   L.off_a = L.off_m + align256(L.nchunk * C * 4);
@@ -1812,10 +1950,9 @@ int64_t split_ws_need(int64_t ntok, int C, int ntarg) {
   int nt, ntiles;
   int64_t total;
   split_items(C, ntarg, &nt, &ntiles, &total);
-  int tail = 0, S = 1;
   const int64_t ntok_p = ((ntok + XTOK - 1) / XTOK) * XTOK;
-  tail_split(total, ntok_p / 16, split_slots(), 16, &tail, &S);
-  return split_layout(ntok, C, ntarg, tail, S).bytes;
+  const TailPlan P = split_tail(total, total - (int64_t)nt * ntarg, ntok_p / 16, split_slots(), INT64_MAX);
+  return split_layout(ntok, C, ntarg, P.slots()).bytes;
 }
 
 // Whole items per launch of the split kernel, in rounds of `slots` workgroups (see launch_split).
@@ -1828,6 +1965,16 @@ int64_t split_ws_need(int64_t ntok, int C, int ntarg) {
 // -0.2 % with 3 / 5 rounds on the other box.
 constexpr int XSEG_ROUNDS = 1;
 
+// The reduction of the tail's partial tiles (none when every item ran whole).
+int launch_split_reduce(const float* wsf, const TailPlan& P, int64_t nks, int full, int ntarg, int nt, int C,
+                        int circ, const float* scale, const float* rsc, const HTargets& tg, hipStream_t s) {
+  if (P.slots() == 0) return RQ_OK;
+  hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)P.items(), 16), dim3(XTHREADS), 0, s, wsf, P, nks, full, ntarg, nt,
+                     C, circ, scale, rsc, tg);
+  RQ_CHECK_LAUNCH();
+  return RQ_OK;
+}
+
 int launch_split(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C, const HTargets& tg,
                  int ntarg, void* ws, int64_t ws_bytes, hipStream_t s) {
   int nt, ntiles;
@@ -1835,16 +1982,12 @@ int launch_split(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C, c
   split_items(C, ntarg, &nt, &ntiles, &total);
   if (total > 0x7fffffff / 8) return RQ_EINVAL;
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && (((size_t)ldx * 2) % 16 == 0);
-  int tail = 0, S = 1;
-  SplitLayout L = split_layout(ntok, C, ntarg, 0, 1);
+  SplitLayout L = split_layout(ntok, C, ntarg, 0);
   const int64_t nks = L.ntok_p / 16;
-  tail_split(total, nks, split_slots(), 16, &tail, &S);
-  L = split_layout(ntok, C, ntarg, tail, S);
-  if (ws_bytes < L.bytes) {                       // no room for the slices: whole items only
-    tail = 0;
-    S = 1;
-    L = split_layout(ntok, C, ntarg, 0, 1);
-  }
+  // slices as far as the workspace has room for their partial tiles
+  const TailPlan P = split_tail(total, total - (int64_t)nt * ntarg, nks, split_slots(),
+                                (ws_bytes - L.bytes) / ((int64_t)XPART * 4));
+  L = split_layout(ntok, C, ntarg, P.slots());
   char* wb = reinterpret_cast<char*>(ws);
   uint16_t* xt = reinterpret_cast<uint16_t*>(wb + L.off_xt);
   float* sT = reinterpret_cast<float*>(wb + L.off_st);
@@ -1866,9 +2009,8 @@ int launch_split(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C, c
     const int rc = launch_act_square(x, x_dtype, ntok, ldx, C, tg, ntarg, apart, wb + act_off(), s);
     if (rc) return rc;
   }
-  const int full = (int)(total - tail);
-  int* cnt = tail > 0 ? reinterpret_cast<int*>(ws) : nullptr;
-  float* wsf = tail > 0 ? reinterpret_cast<float*>(wb + L.off_part) : nullptr;
+  const int full = (int)(total - P.items());
+  float* wsf = reinterpret_cast<float*>(wb + L.off_part);
   const int od_items = nt * (nt - 1) / 2 * ntarg;
   // Segments of XSEG_ROUNDS rounds of whole items, each a launch of its own (the tail's slices
   // ride with the last): the kernel boundary brings every XCD's workgroups back in step.
@@ -1882,17 +2024,21 @@ int launch_split(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C, c
     const int p1 = (q + 1 == nseg) ? full : (int)((int64_t)rounds * (q + 1) / nseg) * slots;
     const int segn = p1 - p0;
     const int od_seg = std::min(segn, std::max(0, od_items - p0));
-    const dim3 grid((unsigned)(segn + (q + 1 == nseg ? (int64_t)tail * S : 0)));
+    const dim3 grid((unsigned)(segn + (q + 1 == nseg ? P.wgs() : 0)));
     if (x_dtype == RQ_F16 && g_hmath.load() == RQ_HMATH_SPLIT16X3)
       hipLaunchKernelGGL((k_hessian_split<__half, 3>), grid, block, 0, s, xt, C, sT, L.ntok_p, scale, tg, ntarg,
-                         nt, ntiles, nks, p0, segn, od_seg, full, S, wsf, cnt);
+                         nt, ntiles, nks, p0, segn, od_seg, full, P, wsf);
     else if (x_dtype == RQ_F16)
       hipLaunchKernelGGL((k_hessian_split<__half, 2>), grid, block, 0, s, xt, C, sT, L.ntok_p, scale, tg, ntarg,
-                         nt, ntiles, nks, p0, segn, od_seg, full, S, wsf, cnt);
+                         nt, ntiles, nks, p0, segn, od_seg, full, P, wsf);
     else
       hipLaunchKernelGGL((k_hessian_split<__hip_bfloat16, 3>), grid, block, 0, s, xt, C, sT, L.ntok_p, scale, tg,
-                         ntarg, nt, ntiles, nks, p0, segn, od_seg, full, S, wsf, cnt);
+                         ntarg, nt, ntiles, nks, p0, segn, od_seg, full, P, wsf);
     RQ_CHECK_LAUNCH();
+  }
+  {
+    const int rc = launch_split_reduce(wsf, P, nks, full, ntarg, nt, C, 1, scale, nullptr, tg, s);
+    if (rc) return rc;
   }
   if (stop && hipEventRecord(stop, s) != hipSuccess) return RQ_EHIP;
   return RQ_OK;
@@ -1905,9 +2051,9 @@ struct SplitLayout32 {
   int64_t off_xh, off_xl, off_xc, off_rs, bytes;
 };
 
-SplitLayout32 split_layout32(int64_t ntok, int C, int ntarg, int64_t tail, int S) {
+SplitLayout32 split_layout32(int64_t ntok, int C, int ntarg, int64_t parts) {
   SplitLayout32 L;
-  L.base = split_layout(ntok, C, ntarg, tail, S);
+  L.base = split_layout(ntok, C, ntarg, parts);
   const int64_t frag16 = align256((int64_t)((C + 31) / 32) * 32 * L.base.ntok_p * 2);
   L.off_xh = L.base.bytes;
   L.off_xl = L.off_xh + frag16;
@@ -1923,10 +2069,9 @@ int64_t split32_ws_need(int64_t ntok, int C, int ntarg) {
   int nt, ntiles;
   int64_t total;
   split_items(C, ntarg, &nt, &ntiles, &total);
-  int tail = 0, S = 1;
   const int64_t ntok_p = ((ntok + XTOK - 1) / XTOK) * XTOK;
-  tail_split(total, ntok_p / 16, split32_slots(), 16, &tail, &S);
-  return split_layout32(ntok, C, ntarg, tail, S).bytes;
+  const TailPlan P = split_tail(total, total - (int64_t)nt * ntarg, ntok_p / 16, split32_slots(), INT64_MAX);
+  return split_layout32(ntok, C, ntarg, P.slots()).bytes;
 }
 
 int launch_split32(const float* x, int64_t ntok, int64_t ldx, int C, const HTargets& tg, int ntarg, void* ws,
@@ -1936,16 +2081,12 @@ int launch_split32(const float* x, int64_t ntok, int64_t ldx, int C, const HTarg
   split_items(C, ntarg, &nt, &ntiles, &total);
   if (total > 0x7fffffff / 8) return RQ_EINVAL;
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && (((size_t)ldx * 4) % 16 == 0);
-  int tail = 0, S = 1;
-  SplitLayout32 L = split_layout32(ntok, C, ntarg, 0, 1);
+  SplitLayout32 L = split_layout32(ntok, C, ntarg, 0);
   const int64_t nks = L.base.ntok_p / 16;
-  tail_split(total, nks, split32_slots(), 16, &tail, &S);
-  L = split_layout32(ntok, C, ntarg, tail, S);
-  if (ws_bytes < L.bytes) {                       // no room for the slices: whole items only
-    tail = 0;
-    S = 1;
-    L = split_layout32(ntok, C, ntarg, 0, 1);
-  }
+  // slices as far as the workspace has room for their partial tiles
+  const TailPlan P = split_tail(total, total - (int64_t)nt * ntarg, nks, split32_slots(),
+                                (ws_bytes - L.bytes) / ((int64_t)XPART * 4));
+  L = split_layout32(ntok, C, ntarg, P.slots());
   char* wb = reinterpret_cast<char*>(ws);
   uint16_t* xh = reinterpret_cast<uint16_t*>(wb + L.off_xh);
   uint16_t* xl = reinterpret_cast<uint16_t*>(wb + L.off_xl);
@@ -1971,14 +2112,17 @@ int launch_split32(const float* x, int64_t ntok, int64_t ldx, int C, const HTarg
     const int rc = launch_act_square(x, RQ_F32, ntok, ldx, C, tg, ntarg, apart, wb + act_off(), s);
     if (rc) return rc;
   }
-  const int full = (int)(total - tail);
-  int* cnt = tail > 0 ? reinterpret_cast<int*>(ws) : nullptr;
-  float* wsf = tail > 0 ? reinterpret_cast<float*>(wb + L.base.off_part) : nullptr;
-  dim3 grid((unsigned)(full + (int64_t)tail * S)), block(XTHREADS);
+  const int full = (int)(total - P.items());
+  float* wsf = reinterpret_cast<float*>(wb + L.base.off_part);
+  dim3 grid((unsigned)(full + P.wgs())), block(XTHREADS);
   hipEvent_t stop = timing_begin(s);
   hipLaunchKernelGGL(k_hessian_split32, grid, block, 0, s, xh, xl, xc, C, sT, L.base.ntok_p, scale, rs, tg, ntarg,
-                     nt, ntiles, nks, full, S, wsf, cnt);
+                     nt, ntiles, nks, full, P, wsf);
   RQ_CHECK_LAUNCH();
+  {
+    const int rc = launch_split_reduce(wsf, P, nks, full, ntarg, nt, C, 0, scale, rs, tg, s);
+    if (rc) return rc;
+  }
   if (stop && hipEventRecord(stop, s) != hipSuccess) return RQ_EHIP;
   return RQ_OK;
 }
@@ -1987,12 +2131,12 @@ int launch_hessian(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C,
                    int ntarg, void* ws, int64_t ws_bytes, hipStream_t s) {
   const bool aligned = ws && ((reinterpret_cast<uintptr_t>(ws) & 255) == 0);
   if (x_dtype != RQ_F32 && g_hmath.load() != RQ_HMATH_FP32 && aligned &&
-      ws_bytes >= split_layout(ntok, C, ntarg, 0, 1).bytes)
+      ws_bytes >= split_layout(ntok, C, ntarg, 0).bytes)
     return launch_split(x, x_dtype, ntok, ldx, C, tg, ntarg, ws, ws_bytes, s);
   // fp32 X: the split kernel (products within ~2^-20.5) only in the opt-in two-piece mode; by
   // default the fp32 MFMA kernel below forms the reference's products exactly
   if (x_dtype == RQ_F32 && g_hmath.load() == RQ_HMATH_SPLIT16 && aligned &&
-      ws_bytes >= split_layout32(ntok, C, ntarg, 0, 1).bytes)
+      ws_bytes >= split_layout32(ntok, C, ntarg, 0).bytes)
     return launch_split32(static_cast<const float*>(x), ntok, ldx, C, tg, ntarg, ws, ws_bytes, s);
   const int nt = (C + HT - 1) / HT;
   const int ntiles = nt * (nt + 1) / 2;
@@ -2112,7 +2256,7 @@ extern "C" int rq_hessian_accum_noalloc(const void* x, int x_dtype, int64_t ntok
   // the least scratch the kernel rq_hessian_accum would choose needs (whole items only)
   const int n = G < HMAXT ? G : HMAXT;
   const int64_t need = (x_dtype != RQ_F32 && g_hmath.load() != RQ_HMATH_FP32)
-                           ? split_layout(ntok, C, n, 0, 1).bytes
+                           ? split_layout(ntok, C, n, 0).bytes
                            : hessian_ws_bytes(ntok, C, 0, 1);
   if (need > (int64_t)RQ_NOALLOC_SCRATCH_BYTES) return RQ_EINVAL;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -248,3 +248,30 @@ def test_split_fp32_x_deterministic_nonfinite_and_multi_target():
         iu2 = torch.triu_indices(640, 640)
         # (another target count splits the tail into other token slices: fp32 sums in another order)
         assert rel_fro(_upper(Hm[t], iu2), _upper(H, iu2)) <= 1e-6 and torch.equal(am[t], ac)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,C,G", [(2561, 700, 30),      # 90 + 90 items, whole diagonal tiles, ranges
+                                   (6400, 1024, 10),     # 60 + 40 items, 2 diagonal slices, ranges
+                                   (2048, 1000, 32),     # a whole round, then 64 diagonal items
+                                   (300, 513, 2), (16, 257, 3)])
+def test_split_tail_ranges(n, C, G, dtype):
+    """Tails cut into ranges that cross items, diagonal tiles whole or in slices, blocks below a
+    diagonal tile's diagonal written transposed, ragged edges: within 1e-6 of the fp64 sum as the
+    whole tiles are, the same twice, and H's other contents kept (H += on a non-zero H)."""
+    g = torch.Generator(device=DEV).manual_seed(n + C)
+    x = torch.randn((n, C), device=DEV, generator=g).to(dtype)
+    s = torch.randn((n, G), device=DEV, generator=g).exp_()
+    H0 = torch.randn((G, C, C), device=DEV, generator=g)
+    outs = []
+    for _ in range(2):
+        H, a = H0.clone(), torch.zeros(C, device=DEV)
+        K.hessian_accum(x, s, H, a)
+        outs.append((H, a))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    xd = x.double()
+    iu = torch.triu_indices(C, C, device=DEV)
+    for t in range(G):
+        ref = H0[t].double() + xd.t().contiguous() @ (xd * s[:, t:t + 1].double())
+        got, ref = outs[0][0][t].double()[iu[0], iu[1]], ref[iu[0], iu[1]]
+        assert float((got - ref).norm() / ref.norm()) <= 1e-6
