@@ -825,3 +825,69 @@ def test_find_params_mse_widths(n, gs, sym):
         for i in torch.nonzero(~same).flatten().tolist():
             e_gpu, e_ora = clip_err(Wg[i], sg[i], zg[i]), clip_err(Wg[i], so[i], zo[i])
             assert abs(e_gpu - e_ora) <= 2.0 ** -13 * e_ora, (i, e_gpu, e_ora)
+
+
+@pytest.mark.parametrize("case", ["plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "inf_w", "nan_w", "big_w"])
+@pytest.mark.parametrize("count", [128, 100, 17])
+@pytest.mark.parametrize("atomic", [False, True])
+def test_quant_block_divides(case, count, atomic):
+    """The column loop's residual divides and the IEEE divide it falls back to: codes and errors equal
+    the reference's operations in fp32, one rounding each (no tolerance), for weights, steps and
+    diagonals in and out of the residual divide's range and for blocks narrower than the kernel's.
+    (Zeros of either sign are equal.)"""
+    if atomic and case in ("inf_w", "nan_w", "small_diag"):
+        pytest.skip("the solve's order of NaN and infinity is not pinned (diagonals of 1e-20 overflow it)")
+    r = rng(count + len(case))
+    R, C = 40, count
+    W = torch.from_numpy(r.standard_normal((R, C)).astype(np.float32) * 0.02)
+    U = torch.from_numpy(np.triu(r.standard_normal((C, C)) * 0.05).astype(np.float32))
+    U.diagonal().copy_(torch.from_numpy(r.uniform(0.5, 2.0, C).astype(np.float32)))
+    scale = torch.from_numpy(r.uniform(0.004, 0.006, R).astype(np.float32))
+    if case == "tiny_w":
+        W[::3] *= 1e-32
+        W[1::3] = 0
+    elif case == "tiny_scale":
+        scale[::4] = 3e-21
+    elif case == "wide_scale":
+        scale[::4] = 1e25
+    elif case == "small_diag":
+        U.diagonal()[::16] = 1e-20
+    elif case == "inf_w":
+        W[3, C // 2] = float("inf")
+    elif case == "nan_w":
+        W[3, C // 2] = float("nan")
+    elif case == "big_w":
+        W[5] *= 1e25
+    maxq = 7
+    wc, codes, errs = W.clone(), torch.zeros(R, C), torch.zeros(R, C)
+    if atomic:
+        codes = torch.clamp(torch.round(wc / scale[:, None]), -(maxq + 1), maxq)
+        res = (wc - scale[:, None] * codes).double()
+        for i in range(C):
+            e = (res[:, i].float() * (1.0 / U[i, i])).double()
+            errs[:, i] = e.float()
+            # one fused multiply-add: exact product and sum in fp64 up to its own rounding
+            res[:, i + 1:] = (res[:, i + 1:] - e[:, None] * U[i, i + 1:].double()).float().double()
+    else:
+        for i in range(C):
+            x = wc[:, i]
+            codes[:, i] = torch.clamp(torch.round(x / scale), -(maxq + 1), maxq)
+            e = (x - scale * codes[:, i]) / U[i, i]
+            errs[:, i] = e
+            wc[:, i:] -= e[:, None] * U[i, i:][None]
+    dW, dU = W.to(DEV).contiguous(), U.to(DEV)[None].contiguous()
+    z = torch.zeros(R, C, device=DEV)
+    out = torch.empty((R, C), dtype=torch.int16, device=DEV)
+    err = torch.zeros((R, count), device=DEV)
+    K.quant_block(dW, dU, z, z, R, 0, count, nat.RQ_QMODE_CHANNEL, scale.to(DEV), None, None, maxq, True, atomic,
+                  torch.zeros(1, dtype=torch.int32, device=DEV), out, err)
+    torch.cuda.synchronize()
+    want = torch.where(codes.isnan(), torch.full_like(codes, -32768.0), codes)
+    got, e_got = out.cpu().float(), err.cpu()
+    if atomic:
+        # (the fp64 stand-in for a fused multiply-add rounds twice once in 2^29)
+        assert torch.equal(got, want)
+        assert float((e_got.double() - errs.double()).norm()) <= 1e-6 * float(errs.double().norm())
+    else:
+        assert torch.equal(got, want)
+        assert torch.equal(e_got.nan_to_num(123.0), errs.nan_to_num(123.0))
