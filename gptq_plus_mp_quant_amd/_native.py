@@ -56,6 +56,7 @@ SIGNATURES = {
                             _I, _P, _P, _P, _I, _P, _L, _P, _D, _P]),
     "rq_quant_block_lookahead": (_I, [_P, _L, _P, _I, _I, _I, _I, _I, _P, _I, _I, _P, _P, _P, _I, _I, _I, _P,
                                       _P, _P]),
+    "rq_block_loop": (_I, [_P, _L, _P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _I, _P, _P, _L, _P]),
     "rq_trailing_update": (_I, [_P, _L, _P, _P, _L, _P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _L,
                                 _P, _D, _P]),
     "rq_writeback": (_I, [_P, _I, _I, _P, _I, _P, _P, _P, _I, _P, _I, _L, _P, _P, _P, _P]),

@@ -44,6 +44,7 @@
 // :1500-1511), the GH update itself is unchanged; in block_gd the whole W update is scaled by
 // second_order_scale (:1546-1549).  k_trailing (fp32 16x16x4 MFMA, 64x64 tiles) takes the
 // shapes those two cannot (a block width that is not a multiple of 8, unaligned operands).
+#include <algorithm>
 #include <type_traits>
 
 #include "rq_common.h"
@@ -90,6 +91,7 @@ struct QBArgs {
   const int* z_nonzero;
   int16_t* codes;
   float* err;
+  int64_t lde;                // row stride of err
   const float* anchor;
   int64_t lda;
   const float* beta;
@@ -97,7 +99,8 @@ struct QBArgs {
   // Look-ahead launch (k_block_lookahead): the previous block's update of this block's
   // columns, applied by each workgroup to its own rows before the column loop; zero_terms: Z
   // (hence GH) is identically zero, z_nonzero is not read.
-  const float* near_err;      // err of the previous block [R, near_count], or NULL
+  const float* near_err;      // err of the previous block (row stride near_lde), or NULL
+  int64_t near_lde;
   int near_i1, near_count;
   int zero_terms;
 };
@@ -177,7 +180,7 @@ __device__ __forceinline__ void quant_block_body(const QBArgs& a, int bx, int by
     for (int e = tid; e < (256 / QL) * pc; e += 256) {
       const int rl = e / pc, kk = e % pc;
       const int rr = bx * (256 / QL) + rl;
-      Ep[rl * QB_MAXB + kk] = (rr < a.R_s) ? a.near_err[(int64_t)(sub * a.R_s + rr) * pc + kk] : 0.0f;
+      Ep[rl * QB_MAXB + kk] = (rr < a.R_s) ? a.near_err[(int64_t)(sub * a.R_s + rr) * a.near_lde + kk] : 0.0f;
     }
     __syncthreads();
     float acc[NS];
@@ -290,7 +293,7 @@ __device__ __forceinline__ void quant_block_body(const QBArgs& a, int bx, int by
   __syncthreads();
 
   int16_t* crow = a.codes + (int64_t)row * a.C + i1;
-  float* erow = a.err + (int64_t)row * count;
+  float* erow = a.err + (int64_t)row * a.lde;
   // row i of the block for this lane: h[k] = Hinv1[i][16 k + t]
   auto hrow = [&](int i, float (&h)[NS]) __attribute__((always_inline)) {
 #pragma unroll
@@ -598,17 +601,38 @@ constexpr int TSTAGE = TA_BYTES + 4 * THROW;
 
 typedef float floatx32 __attribute__((ext_vector_type(32)));
 
+// A uniform pointer and a lane's byte offset: one scalar address and one 32-bit vector register for
+// every access of a kind, instead of 64-bit vector arithmetic per access.  Vector instructions
+// issue at a third of their rate while an fp32 MFMA runs on the SIMD (17 cycles against 6 between
+// dependent ones).  With the loop over blocks in one call, a look-ahead launch: 58.2 -> 52.3 us at
+// R = C = 4096 and 134.6 -> 123.3 us at 4096 x 14336 (the residual divides included); classic
+// GPTQ at 1024 x 4096 41.6 (two launches a block) -> 30.6 us.
+template <typename T>
+__device__ __forceinline__ T* at_bytes(T* base, uint32_t off) {
+  asm("" : "+s"(base));                // (left alone, the compiler adds the two in vector registers)
+  typedef typename std::conditional<std::is_const<T>::value, const char, char>::type B;
+  return reinterpret_cast<T*>(reinterpret_cast<B*>(base) + off);
+}
+
 struct TwArgs {
   float* Wp;
   int64_t ldw;
   const float* Hinv;
   int C, R_s, i1, count;
-  const float* err;
+  const float* err;      // row stride lde
   float f;               // 1, or second_order_scale (RQ_GMODE_BLOCK_GD)
-  int nrt, nct;          // row tiles per subgroup, column tiles
-  int total;             // nrt * nct * subgroups
+  int nrt, nsub;         // row tiles per subgroup, subgroups
   int cbeg;              // first updated column (i1 + count; later in a look-ahead launch)
+  int total;             // row tiles x column tiles x subgroups
+  int64_t lde;
 };
+
+TwArgs tw_args(float* Wp, int64_t ldw, const float* Hinv, int C, int R, int R_s, int i1, int count, const float* err,
+               int64_t lde, float f, int cbeg) {
+  TwArgs w{Wp, ldw, Hinv, C, R_s, i1, count, err, f, (R_s + TT - 1) / TT, R / R_s, cbeg, 0, lde};
+  w.total = C > cbeg ? w.nrt * w.nsub * ((C - cbeg + TT - 1) / TT) : 0;
+  return w;
+}
 
 struct TStages {
   uint8_t* s[TSTAGES];
@@ -622,15 +646,16 @@ __device__ __forceinline__ void lds_dma16(const void* g, uint8_t* l) {
 #define TWAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
 
 struct TwTile {
-  const float* srcA;
+  const float* srcA;       // wave-uniform bases, and this lane's byte offsets from them
   const float* srcB;
+  uint32_t voffA, voffB;
   int wave, wc, aoff0, aoff1, boff, nk;
   int64_t ldh;
   floatx32 acc[2];
 
   __device__ __forceinline__ void stage(uint8_t* st, int kt) {
-    lds_dma16(srcA + kt * 8, st + wave * TCH);
-    lds_dma16(srcB + (int64_t)kt * 8 * ldh, st + TA_BYTES + wave * THROW);
+    lds_dma16(at_bytes(srcA + kt * 8, voffA), st + wave * TCH);
+    lds_dma16(at_bytes(srcB + (int64_t)kt * 8 * ldh, voffB), st + TA_BYTES + wave * THROW);
   }
   // Step kt: wait for this wave's 2 staging loads of kt (the TSTAGES-2 later steps may be in
   // flight), meet the other waves (their parts are in LDS, and every read of the FILL stage,
@@ -666,11 +691,11 @@ __device__ __forceinline__ void trailing_w_body(const TwArgs& a, int b, const TS
   // tiles of one Hinv column strip meet in one L2.
   const int per = a.total / 8, rem8 = a.total % 8;
   const int xcd = b % 8, idx = b / 8;
-  const int t = (xcd < rem8) ? xcd * (per + 1) + idx : rem8 * (per + 1) + (xcd - rem8) * per + idx;
-  if (t >= a.total) return;
-  const int per_sub = a.nrt * a.nct;
-  const int sub = t / per_sub, u = t % per_sub;
-  const int ct = u / a.nrt, rt = u % a.nrt;
+  if (b >= a.total) return;
+  const int t = xcd * per + min(xcd, rem8) + idx;
+  const int per_sub = a.total / a.nsub, u = t % per_sub;
+  const int sub = __builtin_amdgcn_readfirstlane(t / per_sub);
+  const int ct = __builtin_amdgcn_readfirstlane(u / a.nrt), rt = __builtin_amdgcn_readfirstlane(u % a.nrt);
   const int rl0 = rt * TT, c0 = a.cbeg + ct * TT;
   const int64_t rbase = (int64_t)sub * a.R_s;
 
@@ -686,10 +711,12 @@ __device__ __forceinline__ void trailing_w_body(const TwArgs& a, int b, const TS
     // 2 wave, 2 wave + 1 (columns clamped to a whole in-bounds quad)
     const int rho = lane >> 1, q = (lane & 1) ^ ((rho >> 3) & 1);
     const int rl = min(rl0 + 32 * w.wave + rho, a.R_s - 1);
-    w.srcA = a.err + (rbase + rl) * a.count + 4 * q;
+    w.srcA = a.err + (rbase + rl0) * a.lde;
+    w.voffA = (uint32_t)((rl - rl0) * (int)a.lde + 4 * q) * 4u;
     const int kr = 2 * w.wave + (lane >> 5);
     const int c = min(c0 + 4 * (lane & 31), a.C - 4);
-    w.srcB = a.Hinv + (int64_t)sub * a.C * a.C + (int64_t)(a.i1 + kr) * a.C + c;
+    w.srcB = a.Hinv + (int64_t)sub * a.C * a.C + (int64_t)a.i1 * a.C + c0;
+    w.voffB = (uint32_t)(kr * a.C + c - c0) * 4u;
   }
   // err of this lane: wave row `lane` = tile row 64 wr + lane, in chunk 2 wr + lane / 32 at
   // in-chunk row rho = lane % 32; k quad q sits at slot 2 rho + (q ^ ((rho / 8) % 2))
@@ -706,18 +733,32 @@ __device__ __forceinline__ void trailing_w_body(const TwArgs& a, int b, const TS
 #pragma unroll
     for (int e = 0; e < 32; ++e) w.acc[h][e] = 0.0f;
 
-  // This lane's 64 outputs of W (clamped in-bounds addresses), loaded before the staging so
-  // their latency overlaps the first stage's: output e of half h is wave row
-  // 32 (e / 16) + 8 ((e % 16) / 4) + 4 (lane / 32) + e % 4, wave column 32 h + lane % 32.
+  // This lane's 64 outputs of W: output e of half h is wave row
+  // 32 (e / 16) + 8 ((e % 16) / 4) + 4 (lane / 32) + e % 4, wave column 32 h + lane % 32; loaded
+  // before the staging so their latency overlaps the first stage's.
   const int rw0 = rl0 + 64 * wr + 4 * (lane >> 5), cw0 = c0 + 64 * w.wc + (lane & 31);
+  const bool full = (rl0 + TT <= a.R_s) && (c0 + TT <= a.C);
+  float* wbase = a.Wp + (rbase + rl0 + 64 * wr) * a.ldw + c0 + 64 * w.wc;
+  const uint32_t wvoff = (uint32_t)(4 * (lane >> 5) * (int)a.ldw + (lane & 31)) * 4u;
   float wv[2][32];
+  if (full) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int e = 0; e < 32; ++e) {
-      const int rl = min(rw0 + 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4), a.R_s - 1);
-      wv[h][e] = a.Wp[(rbase + rl) * a.ldw + min(cw0 + 32 * h, a.C - 1)];
-    }
+      for (int e = 0; e < 32; ++e) {
+        const int dr = 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4);
+        wv[h][e] = *at_bytes(wbase + dr * a.ldw + 32 * h, wvoff);
+      }
+    asm volatile("" ::: "memory");     // (not merged with the other branch's loads: vector addresses)
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int rl = min(rw0 + 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4), a.R_s - 1);
+        wv[h][e] = a.Wp[(rbase + rl) * a.ldw + min(cw0 + 32 * h, a.C - 1)];
+      }
+  }
 
   static_assert(TSTAGES == 4, "unrolled stage schedule");
 #pragma unroll
@@ -736,17 +777,32 @@ __device__ __forceinline__ void trailing_w_body(const TwArgs& a, int b, const TS
   TWAIT_VM(0);   // no staging in flight when the workgroup ends
 
   // W - tot, or W - f * tot (block_gd), into the prefetched outputs.
-  const bool full = (rl0 + TT <= a.R_s) && (c0 + TT <= a.C);
   const bool scaled = a.f != 1.0f;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int e = 0; e < 32; ++e) {
-      const int rl = rw0 + 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4), c = cw0 + 32 * h;
       const float tot = w.acc[h][e];
-      const float v = wv[h][e] - (scaled ? a.f * tot : tot);
-      if (full || (rl < a.R_s && c < a.C)) a.Wp[(rbase + rl) * a.ldw + c] = v;
+      wv[h][e] = wv[h][e] - (scaled ? a.f * tot : tot);
     }
+  if (full) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int dr = 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4);
+        *at_bytes(wbase + dr * a.ldw + 32 * h, wvoff) = wv[h][e];
+      }
+    asm volatile("" ::: "memory");
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const int dr = 32 * (e / 16) + 8 * ((e % 16) / 4) + (e % 4);
+        if (rw0 + dr < a.R_s && cw0 + 32 * h < a.C) a.Wp[(rbase + rw0 + dr) * a.ldw + cw0 + 32 * h] = wv[h][e];
+      }
+  }
 }
 
 __global__ __launch_bounds__(256, 2) void k_trailing_w(TwArgs a) {
@@ -763,7 +819,8 @@ __global__ __launch_bounds__(256, 2) void k_trailing_w(TwArgs a) {
 // k+1's columns), the others update the columns past block k+1 with block k's err
 // (k_trailing_w's tiles).  The two parts touch disjoint columns and different err buffers,
 // so block k+1's column loop runs while block k's wide update does.  The quantising
-// workgroups come first in the grid, so they are dispatched first.
+// workgroups come first in the grid, so they are dispatched first (alternating them with the
+// tiles measured 53.5 -> 59 us a block at R = C = 4096, 155 -> 170 at R = 14336).
 template <int NS>
 __global__ __launch_bounds__(256, 2) void k_block_lookahead(QBArgs q, TwArgs w, int nqx, int nq) {
   constexpr int QBYTES = qb_lds_bytes<NS>(true);
@@ -948,6 +1005,36 @@ __global__ __launch_bounds__(256, 2) void k_trailing_z(TzArgs a) {
   }
 }
 
+// A frozen-mode block without first-order terms (the caller sets the block's own fields).
+QBArgs plain_block(float* Wp, int64_t ldw, const float* Hinv, int C, int R, int R_s, int qmode, const float* scale,
+                   const int32_t* col_group, int maxq, int sym, int16_t* codes) {
+  QBArgs q{};
+  q.Wp = Wp;
+  q.ldw = ldw;
+  q.Hinv = Hinv;
+  q.C = C;
+  q.ldgh = C;
+  q.R = R;
+  q.R_s = R_s;
+  q.qmode = qmode;
+  q.scale = scale;
+  q.col_group = col_group;
+  q.maxq = (float)maxq;
+  q.sym = sym;
+  q.codes = codes;
+  q.lda = C;
+  q.sos = 1.0f;
+  q.zero_terms = 1;
+  return q;
+}
+
+void launch_lookahead(const QBArgs& q, const TwArgs& w, hipStream_t s) {
+  const int nqx = (q.R_s + 256 / QL - 1) / (256 / QL), nq = nqx * (q.R / q.R_s);
+  const dim3 grid(nq + w.total);
+  if (q.count <= 2 * QL) hipLaunchKernelGGL(k_block_lookahead<2>, grid, dim3(256), 0, s, q, w, nqx, nq);
+  else hipLaunchKernelGGL(k_block_lookahead<8>, grid, dim3(256), 0, s, q, w, nqx, nq);
+}
+
 }  // namespace
 
 extern "C" int rq_quant_block(float* Wp, int64_t ldw, const float* Hinv_all, int C, const float* GH,
@@ -967,7 +1054,7 @@ extern "C" int rq_quant_block(float* Wp, int64_t ldw, const float* Hinv_all, int
   if (qmode == RQ_QMODE_DYNAMIC && !dyn_scale) return RQ_EINVAL;
   if (qmode < 0 || qmode > 2) return RQ_EINVAL;
   QBArgs a{Wp, ldw, Hinv_all, C, GH, Z, ldgh, R, R_s, i1, count, qmode, scale, col_group,
-           dyn_scale, (float)maxq, sym, atomic, z_nonzero, codes, err, anchor, ld_anchor, beta,
+           dyn_scale, (float)maxq, sym, atomic, z_nonzero, codes, err, count, anchor, ld_anchor, beta,
            (float)second_order_scale};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   dim3 grid((R_s + 256 / QL - 1) / (256 / QL), R / R_s), block(256);
@@ -1010,10 +1097,8 @@ extern "C" int rq_trailing_update(float* Wp, int64_t ldw, float* GH, const float
   if (z_zero && (gmode == RQ_GMODE_FROZEN || gmode == RQ_GMODE_BLOCK_GD) && count % 8 == 0 &&
       C % 4 == 0 && i2 % 4 == 0 && al16(Hinv_all) && al16(err)) {
     // Z (and with it GH) identically zero: only W -= f * err Hinv[i1:i2, i2:] remains
-    TwArgs w{Wp, ldw, Hinv_all, C, R_s, i1, count, err,
-             gmode == RQ_GMODE_BLOCK_GD ? (float)second_order_scale : 1.0f,
-             (R_s + TT - 1) / TT, (C - i2 + TT - 1) / TT, 0, i2};
-    w.total = w.nrt * w.nct * (R / R_s);
+    const TwArgs w = tw_args(Wp, ldw, Hinv_all, C, R, R_s, i1, count, err, count,
+                             gmode == RQ_GMODE_BLOCK_GD ? (float)second_order_scale : 1.0f, i2);
     hipLaunchKernelGGL(k_trailing_w, dim3(w.total), dim3(256), 0, s, w);
     RQ_CHECK_LAUNCH();
     return RQ_OK;
@@ -1055,45 +1140,66 @@ extern "C" int rq_quant_block_lookahead(float* Wp, int64_t ldw, const float* Hin
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   // the wide part runs k_trailing_w's tiles: its shape conditions
   if (count % 8 || C % 4 || cbeg % 4 || !al16(Hinv_all) || !al16(err)) return RQ_EINVAL;
-  QBArgs q{};
-  q.Wp = Wp;
-  q.ldw = ldw;
-  q.Hinv = Hinv_all;
-  q.C = C;
-  q.GH = nullptr;
-  q.Z = nullptr;
-  q.ldgh = C;
-  q.R = R;
-  q.R_s = R_s;
+  QBArgs q = plain_block(Wp, ldw, Hinv_all, C, R, R_s, qmode, scale, col_group, maxq, sym, codes);
   q.i1 = i1n;
   q.count = count_next;
-  q.qmode = qmode;
-  q.scale = scale;
-  q.col_group = col_group;
   q.dyn_scale = dyn_scale;
-  q.maxq = (float)maxq;
-  q.sym = sym;
   q.atomic = atomic;
-  q.z_nonzero = nullptr;
-  q.codes = codes;
   q.err = err_next;
-  q.anchor = nullptr;
-  q.lda = C;
-  q.beta = nullptr;
-  q.sos = 1.0f;
+  q.lde = count_next;
   q.near_err = err;
+  q.near_lde = count;
   q.near_i1 = i1;
   q.near_count = count;
-  q.zero_terms = 1;
-  TwArgs w{Wp, ldw, Hinv_all, C, R_s, i1, count, err, 1.0f, (R_s + TT - 1) / TT, (C - cbeg + TT - 1) / TT, 0,
-           cbeg};
-  w.total = (cbeg < C) ? w.nrt * w.nct * (R / R_s) : 0;
-  const int nqx = (R_s + 256 / QL - 1) / (256 / QL), nq = nqx * (R / R_s);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (count_next <= 2 * QL)
-    hipLaunchKernelGGL(k_block_lookahead<2>, dim3(nq + w.total), dim3(256), 0, s, q, w, nqx, nq);
-  else
-    hipLaunchKernelGGL(k_block_lookahead<8>, dim3(nq + w.total), dim3(256), 0, s, q, w, nqx, nq);
+  launch_lookahead(q, tw_args(Wp, ldw, Hinv_all, C, R, R_s, i1, count, err, count, 1.0f, cbeg),
+                   reinterpret_cast<hipStream_t>(stream));
   RQ_CHECK_LAUNCH();
+  return RQ_OK;
+}
+
+// The whole frozen column loop with the GPTQ+ terms identically zero: rq_quant_block for the first
+// block, then one look-ahead launch per block, err alternating between two halves of a row.
+// (Updates of far columns made for four blocks at a time, W read and written once for four
+// chains, measured 10-25 % slower per block than one update per block: the column loop's vector
+// instructions run at a third of their rate beside fp32 MFMAs, and the longer tiles keep those
+// going beside it for longer.)
+extern "C" int rq_block_loop(float* Wp, int64_t ldw, const float* Hinv_all, int C, int R, int R_s, int blocksize,
+                             int qmode, const float* scale, const int32_t* col_group, float* dyn_scale, int maxq,
+                             int sym, int atomic, int16_t* codes, float* err, int64_t lde, void* stream) {
+  if (!Wp || !Hinv_all || !codes || !err) return RQ_EINVAL;
+  if (R <= 0 || R_s <= 0 || R % R_s != 0 || C <= 0 || ldw < C) return RQ_EINVAL;
+  if (blocksize <= 0 || blocksize > QB_MAXB || maxq <= 0 || qmode < 0 || qmode > 2) return RQ_EINVAL;
+  if (qmode == RQ_QMODE_CHANNEL && !scale) return RQ_EINVAL;
+  if (qmode == RQ_QMODE_STATIC && (!scale || !col_group)) return RQ_EINVAL;
+  if (qmode == RQ_QMODE_DYNAMIC && !dyn_scale) return RQ_EINVAL;
+  const int B = blocksize, nb = (C + B - 1) / B;
+  if (lde < 2 * (int64_t)B || lde % 4) return RQ_EINVAL;
+  auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (nb > 1 && (B % 8 || C % 4 || !al16(Hinv_all) || !al16(err))) return RQ_EINVAL;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  QBArgs q = plain_block(Wp, ldw, Hinv_all, C, R, R_s, qmode, scale, col_group, maxq, sym, codes);
+  q.lde = lde;
+  auto block = [&](int k) {
+    q.i1 = k * B;
+    q.count = std::min(B, C - q.i1);
+    q.dyn_scale = dyn_scale ? dyn_scale + (int64_t)k * R : nullptr;
+    q.atomic = atomic && q.i1 + q.count < C;
+    q.err = err + (k % 2) * B;
+  };
+  block(0);
+  const dim3 grid((R_s + 256 / QL - 1) / (256 / QL), R / R_s);
+  if (q.count <= 2 * QL) hipLaunchKernelGGL((k_quant_block<2, 0>), grid, dim3(256), 0, s, q);
+  else hipLaunchKernelGGL((k_quant_block<8, 0>), grid, dim3(256), 0, s, q);
+  RQ_CHECK_LAUNCH();
+  for (int k = 0; k + 1 < nb; ++k) {
+    block(k + 1);
+    q.near_err = err + (k % 2) * B;
+    q.near_lde = lde;
+    q.near_i1 = k * B;
+    q.near_count = B;
+    launch_lookahead(q, tw_args(Wp, ldw, Hinv_all, C, R, R_s, k * B, B, q.near_err, lde, 1.0f,
+                                (int)std::min<int64_t>((int64_t)(k + 2) * B, C)), s);
+    RQ_CHECK_LAUNCH();
+  }
   return RQ_OK;
 }

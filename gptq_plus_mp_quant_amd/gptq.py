@@ -133,9 +133,12 @@ class GPTQ:
         del workspace, H_work
 
         codes = torch.empty((R, C), dtype=torch.int16, device=dev)
-        err = torch.empty((R, min(blocksize, C)), **f32)
+        fused = not dyn_fit and K.block_loop_ok(Hinv_all, C, blocksize)
+        if fused:
+            K.block_loop(Wp, Hinv_all, R, blocksize, qmode, scale_tab, col_group, None, maxq, sym, False, codes)
+        err = None if fused else torch.empty((R, min(blocksize, C)), **f32)
         z_off = torch.zeros(1, dtype=torch.int32, device=dev)      # no first-order term
-        for i1 in range(0, C, blocksize):
+        for i1 in range(0, C, blocksize) if not fused else ():
             i2 = min(i1 + blocksize, C)
             if dyn_fit:
                 for g in range((i1 + groupsize - 1) // groupsize, (i2 + groupsize - 1) // groupsize):

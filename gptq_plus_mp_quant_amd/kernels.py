@@ -327,6 +327,26 @@ def quant_block_lookahead(Wp, Hinv_all, R_s, i1, count, err, count_next, qmode, 
              nat.ptr(err_next), _stream(Wp))
 
 
+def block_loop_ok(Hinv_all, C, blocksize):
+    """Shapes rq_block_loop takes (one block always; else its update tiles' conditions)."""
+    return C <= blocksize or (blocksize % 8 == 0 and C % 4 == 0 and Hinv_all.data_ptr() % 16 == 0)
+
+
+def block_loop(Wp, Hinv_all, R_s, blocksize, qmode, scale, col_group, dyn_scale, maxq, sym, atomic, codes):
+    """The whole frozen column loop with Z identically zero (quant_block and trailing_update for every
+    block, bit for bit); dyn_scale [blocks, R] for dynamic groups."""
+    R, C = Wp.shape
+    if Hinv_all.shape != (R // R_s, C, C) or not Hinv_all.is_contiguous():
+        raise ValueError("block_loop: Hinv_all must be contiguous [G, C, C]")
+    _cout(Wp, "Wp"), _cout(codes, "codes", torch.int16)
+    if dyn_scale is not None and dyn_scale.numel() < -(-C // blocksize) * R:
+        raise ValueError("block_loop: dyn_scale must be [blocks, R]")
+    err = torch.empty((R, -(-blocksize // 2) * 4), dtype=_f32, device=Wp.device)
+    nat.call("rq_block_loop", nat.ptr(Wp), Wp.stride(0), nat.ptr(Hinv_all), C, R, R_s, int(blocksize), int(qmode),
+             nat.ptr(scale), nat.ptr(col_group), nat.ptr(dyn_scale), int(maxq), int(bool(sym)), int(bool(atomic)),
+             nat.ptr(codes), nat.ptr(err), err.stride(0), _stream(Wp))
+
+
 def trailing_update(Wp, GH, Z, Hinv_all, R_s, i1, count, err, z_nonzero, gmode=nat.RQ_GMODE_FROZEN,
                     anchor=None, beta=None, second_order_scale=1.0, z_zero=False):
     """z_zero=True states that Z (and GH) are identically zero, i.e. that z_nonzero holds 0; the

@@ -251,6 +251,17 @@ int rq_quant_block_lookahead(float* Wp, int64_t ldw, const float* Hinv_all, int 
                              int maxq, int sym, int atomic, int16_t* codes, float* err_next,
                              void* stream);
 
+/* The whole column loop of fasterquant (gptq_plus_utils.py:1169-1372, 1500-1570) in frozen mode
+ * with the GPTQ+ terms identically zero: rq_quant_block and rq_trailing_update for every block of
+ * blocksize columns, bit for bit, in one launch per block (block k+1 is quantised while block
+ * k's update runs, rq_quant_block_lookahead).  codes [R, C]; dyn_scale [blocks, R]
+ * (RQ_QMODE_DYNAMIC); err: workspace [R, lde] with lde >= 2 * blocksize, lde % 4 == 0.  atomic: every block but one that ends at C.  More than one
+ * block needs blocksize % 8 == 0, C % 4 == 0 and Hinv_all, err 16-byte aligned (else RQ_EINVAL:
+ * use the two calls). */
+int rq_block_loop(float* Wp, int64_t ldw, const float* Hinv_all, int C, int R, int R_s, int blocksize,
+                  int qmode, const float* scale, const int32_t* col_group, float* dyn_scale, int maxq,
+                  int sym, int atomic, int16_t* codes, float* err, int64_t lde, void* stream);
+
 /* Un-permute and write back -- gptq_plus_utils.py:1850-1875:
  * natural column c of row r takes permuted column j = invperm[c] (identity if NULL):
  * Q = scale(r, j) * code[r, j]; q_out (layer dtype q_dtype, [R, C] row stride ldq) = Q;

@@ -891,3 +891,53 @@ def test_quant_block_divides(case, count, atomic):
     else:
         assert torch.equal(got, want)
         assert torch.equal(e_got.nan_to_num(123.0), errs.nan_to_num(123.0))
+
+
+@pytest.mark.parametrize("G,R_s,C,B,qmode,atomic", [
+    (2, 150, 128 * 11 + 40, 128, "channel", False),   # two whole groups, far columns spread, ragged last block
+    (1, 40, 128 * 9, 128, "static", True),            # far columns of the second window only
+    (3, 136, 128 * 4, 128, "dynamic", False),         # one group, no far columns
+    (2, 64, 32 * 21 + 4, 32, "channel", False),       # narrow blocks: windows of 160 columns
+    (1, 300, 96 * 13, 96, "dynamic", True),           # windows off the tile grid
+    (2, 48, 64 * 18 + 8, 64, "static", False),
+    (2, 24, 24 * 7 + 4, 24, "channel", False),        # blocks that are not grouped
+    (1, 17, 100, 128, "channel", True),               # one block
+    (1, 17, 101, 128, "static", False),
+])
+def test_block_loop_equals_two_calls(G, R_s, C, B, qmode, atomic):
+    """rq_block_loop (updates of far columns made for four blocks at a time) against rq_quant_block +
+    rq_trailing_update for every block: codes, dynamic scales and the working weight bit for bit."""
+    r = rng(170 + C + B)
+    R = G * R_s
+    Hs = torch.stack([_spd(180 + g, C) for g in range(G)]).to(DEV).contiguous()
+    ws = K.chol_workspace(C, DEV, G)
+    Hinv = torch.empty(G, C, C, device=DEV)
+    assert K.chol_hinv_attempt(Hs, [0.01] * G, ws, Hinv).tolist() == [0] * G
+    W0 = torch.from_numpy(r.standard_normal((R, C)).astype(np.float32)).to(DEV)
+    maxq, sym, nblocks = 7, 0, (C + B - 1) // B
+    scale = col_group = None
+    qm = {"channel": nat.RQ_QMODE_CHANNEL, "static": nat.RQ_QMODE_STATIC, "dynamic": nat.RQ_QMODE_DYNAMIC}[qmode]
+    if qmode == "channel":
+        scale = (W0.abs().amax(1) / maxq).contiguous()
+    elif qmode == "static":
+        scale = torch.from_numpy(r.uniform(0.2, 0.6, ((C + 63) // 64, R)).astype(np.float32)).to(DEV).reshape(-1)
+        col_group = (torch.arange(C, device=DEV) // 64).to(torch.int32)
+    zero, nz0 = torch.zeros_like(W0), torch.zeros(1, dtype=torch.int32, device=DEV)
+    Wa, ca = W0.clone(), torch.zeros((R, C), dtype=torch.int16, device=DEV)
+    da = torch.zeros((nblocks, R), device=DEV) if qmode == "dynamic" else None
+    e = torch.empty((R, B), device=DEV)
+    for b, i1 in enumerate(range(0, C, B)):
+        i2 = min(i1 + B, C)
+        K.quant_block(Wa, Hinv, zero, zero, R_s, i1, i2 - i1, qm, scale, col_group, None if da is None else da[b],
+                      maxq, sym, atomic and i2 < C, nz0, ca, e)
+        if i2 < C:
+            K.trailing_update(Wa, zero, zero, Hinv, R_s, i1, i2 - i1, e, nz0, z_zero=True)
+    assert K.block_loop_ok(Hinv, C, B)
+    for _ in range(2):
+        Wb, cb = W0.clone(), torch.zeros((R, C), dtype=torch.int16, device=DEV)
+        db = torch.zeros((nblocks, R), device=DEV) if qmode == "dynamic" else None
+        K.block_loop(Wb, Hinv, R_s, B, qm, scale, col_group, db, maxq, sym, atomic, cb)
+        torch.cuda.synchronize()
+        assert torch.equal(ca, cb), "codes"
+        assert torch.equal(Wa, Wb), "working weight"
+        assert da is None or torch.equal(da, db)
