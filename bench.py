@@ -358,7 +358,7 @@ def roofline(cfg, args, kernel_ms, launches, steps):
     if args.x_fp32:   # fp32 activations: exact on the fp32 kernel, or hi w0 + hi w1 + lo w0 (split16)
         traffic, tsrc = None, "fp32 activations: not measured"
         pieces = 3 if args.hessian_math == "split16" else 1
-        kernel = "k_hessian_split32" if args.hessian_math == "split16" else "k_hessian_accum<float>"
+        kernel = "k_hessian_split32" if args.hessian_math == "split16" else "k_hessian_x32"
     peak = FP16_MFMA_PEAK_TFLOPS if pieces > 1 else FP32_MFMA_PEAK_TFLOPS
     return {"bound": "mfma", "achieved": round(ach, 2), "peak": peak, "unit": "TFLOP/s",
             "frac": round(ach / peak, 4), "traffic": traffic,
@@ -611,6 +611,7 @@ def algorithmic_work(cfg, lookahead=False):
         add("k_xprep", n * 4.0 * ntok * C)                      # X read, the blocked copy written
     add("k_hessian_split", 0.0, float(hessian_flops(cfg)))
     add("k_hessian_accum", 0.0, float(hessian_flops(cfg)))
+    add("k_hessian_x32", 0.0, float(hessian_flops(cfg)))
     return w
 
 
@@ -644,7 +645,7 @@ def stats_table(path, cfg, units, config):
                 tf = fl / (per * 1e-3) / 1e12
                 wtxt = f"{fl / 1e9:.1f} GFLOP" + (f", {b / 1e6:.0f} MB" if b else "")
                 ach = f"{tf:.1f} TF/s" + (f" ({100 * tf / peak:.1f} % of {peak})" if peak else "")
-                if key in ("k_hessian_split", "k_hessian_accum"):
+                if key in ("k_hessian_split", "k_hessian_accum", "k_hessian_x32"):
                     # the live launch time covers one add_batch call, which may span dispatches
                     ach += f"; {per / hessian_calls(cfg):.3f} ms per add_batch call"
                 if b and key in ("k_quant_block", "k_block_lookahead"):

@@ -805,7 +805,8 @@ __device__ __forceinline__ int xcd_run(int b, int n) {
 // an agent-scope fence in every slice); a launch of its own spreads an item over 16 workgroups of
 // 8 accumulator rows.  63 items of 4 slices (C = 1365, G = 3, 2505 tokens): 223 -> 62 + 14 us for
 // the call's product kernels.
-// rsc: fp32 X, the row exponents 2^-ex_i (applied in fp64, exact).
+// scale: the columns' exponents, nullptr for none; rsc: k_hessian_split32's row exponents 2^-ex_i
+// (applied in fp64, exact).
 // circ: a diagonal tile's blocks are numbered as diag_rows does (else block bi is row block bi).
 __global__ __launch_bounds__(XTHREADS) void k_split_reduce(const float* __restrict__ ws, TailPlan P, int64_t nks,
                                                            int full, int ntarg, int nt, int C, int circ,
@@ -866,7 +867,7 @@ __global__ __launch_bounds__(XTHREADS) void k_split_reduce(const float* __restri
     }
     any = true;
   }
-  const float inv = (j < C) ? 1.0f / scale[(int64_t)g * C + j] : 0.0f;
+  const float inv = !scale ? 1.0f : (j < C) ? 1.0f / scale[(int64_t)g * C + j] : 0.0f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int i = R0 + 32 * rb + 8 * ((e0 + e) >> 2) + 4 * fh + (e & 3);
@@ -945,7 +946,7 @@ __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split(
 
 // ---------------------------------------------------------------------------------------------
 // fp32 X (k_hessian_split32, run in the opt-in RQ_HMATH_SPLIT16 mode; by default fp32 X runs on
-// the fp32 MFMA kernel): the same 256 x 256 upper tiles, with x no longer exact in 16 bits.
+// k_hessian_x32 below): the same 256 x 256 upper tiles, with x no longer exact in 16 bits.
 // The row operand is x 2^ex_i written as two fp16 pieces hi + lo (22 of x's 24 bits; k_xrows32),
 // the column operand w = fl32(x * s) 2^e_j is split in the kernel from the exact fp32 x (fp32
 // column fragments, k_xprep32) into w0 + w1 (as the two-piece fp16 mode), and each 16-token
@@ -967,12 +968,13 @@ constexpr int X3_STAGE = X3_SAL + 256;
 
 // Stage step k: hi and lo row fragment w, this wave's fp32 column fragment (two halves), and
 // -- wave 0, lanes 0-3 -- the step's 16 saliencies.  4 staging loads per wave (wave 0: 5).
-__device__ __forceinline__ void stage_step32(uint8_t* st, const uint16_t* ph, const uint16_t* pl,
+// rstep: halves from one step's row fragment to the next.
+__device__ __forceinline__ void stage_step32(uint8_t* st, const uint16_t* ph, const uint16_t* pl, int rstep,
                                              const float* pc, const float* sg, int wave, int lane,
                                              int64_t k) {
   asm volatile("" : "+s"(k));
-  lds_dma16(ph + k * 512, st + X3_HI + wave * 1024);
-  lds_dma16(pl + k * 512, st + X3_LO + wave * 1024);
+  lds_dma16(ph + k * rstep, st + X3_HI + wave * 1024);
+  lds_dma16(pl + k * rstep, st + X3_LO + wave * 1024);
   lds_dma16(pc + k * 512, st + X3_COL + wave * 2048);
   lds_dma16(pc + k * 512 + 256, st + X3_COL + wave * 2048 + 1024);
   if (wave == 0 && lane < 4) lds_dma16(sg + 16 * k + 4 * lane, st + X3_SAL);
@@ -1018,7 +1020,7 @@ __device__ __forceinline__ void split_step32(uint4 (&p)[2], uint4 (&ah)[8], uint
   typedef XType<__half>::v8 v8;
   XWAIT_VM(4 * (X32DEPTH - 3));
   RQ_STAGE_BARRIER();
-  stage_step32(L.s[FILL], ph, pl, pc, sg, wave, lane, min(k + X32DEPTH - 1, last));
+  stage_step32(L.s[FILL], ph, pl, 512, pc, sg, wave, lane, min(k + X32DEPTH - 1, last));
   // phase A: hi rows x (w1, w0); the lo rows of this step and the next column fragment are read
   const uint8_t* cur = static_cast<const uint8_t*>(__builtin_assume_aligned(L.s[CUR] + X3_LO + lane * 16, 16));
 #pragma unroll
@@ -1091,7 +1093,7 @@ __device__ __forceinline__ void split_tile32(const uint16_t* __restrict__ XH, co
 
   const int64_t last = kend - 1;
 #pragma unroll
-  for (int h = 0; h < X32DEPTH - 1; ++h) stage_step32(L.s[h], ph, pl, pc, sg, wave, lane, min(kbeg + h, last));
+  for (int h = 0; h < X32DEPTH - 1; ++h) stage_step32(L.s[h], ph, pl, 512, pc, sg, wave, lane, min(kbeg + h, last));
   uint4 p[2], ah[8], al[8];
   XWAIT_VM(4 * (X32DEPTH - 2));         // this wave's staging of step kbeg
   RQ_STAGE_BARRIER();       // and the other waves'
@@ -1168,6 +1170,175 @@ __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split32(
   };
   const int w = b < full ? -1 : xcd_run(b - full, P.wgs());
   whole_or_tail(tile, b < full ? item_position(b, full, nt * (nt - 1) / 2 * ntarg) : 0, w, P, nks, full, total, ws);
+}
+
+// ---------------------------------------------------------------------------------------------
+// fp32 X by default (k_hessian_x32): the reference's fp32 products on v_mfma_f32_32x32x2f32, with
+// the split kernels' tiles, waves, tail and staging.  k_hessian_accum, which needs no workspace,
+// reads X as it is: every thread 64 bytes of a token, 16 KB from its neighbour's, transposed
+// through LDS a word at a time and weighted in every workgroup.  Here k_xprep32 has written the
+// chunk in fragments once, the ring is filled by direct global->LDS loads, and per 16 tokens a
+// wave issues 64 MFMAs, 20 16-byte LDS reads and 8 multiplications (vector instructions issue at a
+// third of their rate beside fp32 MFMAs).  C = 4096, four targets, 16384 tokens: 8.30 ms at 132 TF/s (84 %
+// of the fp32 MFMA peak, 86 % of a large library product's rate) against k_hessian_accum's 9.94; the
+// pre-pass 0.12 ms against 0.10 of its act_square pass.  Bound by the matrix unit.
+//
+// A lane of a fragment holds tokens 8 h .. 8 h + 7 of its row or column (h = lane / 32, two halves
+// of 4), so MFMA e of a step multiplies tokens e and 8 + e.  LDS stage as k_hessian_split32, with
+// the two halves of the fp32 row fragments in the place of the hi and lo rows.
+template <bool DIAG, int CUR, int NXT, int FILL>
+__device__ __forceinline__ void x32_step(float (&w)[8], floatx16 (&acc)[XBLK<DIAG>], const XStages& L,
+                                         const float* pr, const float* pc, const float* sg, int wave, int lane,
+                                         int64_t k, int64_t last, int cbw, int lim) {
+  XWAIT_VM(4 * (X32DEPTH - 3));           // this step's and the next one's staging
+  RQ_STAGE_BARRIER();
+  stage_step32(L.s[FILL], reinterpret_cast<const uint16_t*>(pr), reinterpret_cast<const uint16_t*>(pr + 256), 1024,
+               pc, sg, wave, lane, min(k + X32DEPTH - 1, last));
+  const uint8_t* cur = static_cast<const uint8_t*>(__builtin_assume_aligned(L.s[CUR] + lane * 16, 16));
+  constexpr int NP = (XBLK<DIAG> + 1) / 2;
+  float4 f[2][4];                         // a pair's row fragments: [block][half], two pairs in flight
+  auto rows = [&](int j, float4 (&r)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (2 * j + q < XBLK<DIAG>) {
+        const uint8_t* src = cur + diag_rows<DIAG>(cbw, 2 * j + q) * 1024;
+        r[2 * q] = *reinterpret_cast<const float4*>(src + X3_HI);
+        r[2 * q + 1] = *reinterpret_cast<const float4*>(src + X3_LO);
+      }
+  };
+  rows(0, f[0]);
+  float x[8], sv[8];
+  read_col32(L.s[NXT], wave, lane, x, sv);
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    if (DIAG && 2 * j >= lim) break;
+    if (j + 1 < NP) rows(j + 1, f[(j + 1) & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    const float4(&r)[4] = f[j & 1];
+    const float a0[8] = {r[0].x, r[0].y, r[0].z, r[0].w, r[1].x, r[1].y, r[1].z, r[1].w};
+    const float a1[8] = {r[2].x, r[2].y, r[2].z, r[2].w, r[3].x, r[3].y, r[3].z, r[3].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      acc[2 * j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], w[e], acc[2 * j], 0, 0, 0);
+      if (2 * j + 1 < XBLK<DIAG>)
+        acc[2 * j + 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], w[e], acc[2 * j + 1], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) w[e] = x[e] * sv[e];       // fl32(x * s): the reference's `weighted`
+}
+
+template <bool DIAG, int... J>
+__device__ __forceinline__ void x32_round(float (&w)[8], floatx16 (&acc)[XBLK<DIAG>], const XStages& L,
+                                          const float* pr, const float* pc, const float* sg, int wave, int lane,
+                                          int64_t k, int64_t last, int cbw, int lim, int nsteps,
+                                          std::integer_sequence<int, J...>) {
+  ((J < nsteps ? x32_step<DIAG, J, (J + 1) % X32DEPTH, (J + X32DEPTH - 1) % X32DEPTH>(
+                     w, acc, L, pr, pc, sg, wave, lane, k + J, last, cbw, lim)
+               : void()),
+   ...);
+}
+
+template <bool DIAG>
+__device__ __forceinline__ void x32_tile(const float* __restrict__ XC, int64_t nks, int C,
+                                         const float* __restrict__ sg, float* __restrict__ Hg, int R0, int C0,
+                                         int64_t kbeg, int64_t kend, float* __restrict__ part, const XStages& L) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, fh = lane >> 5;
+  const int cbw = split_colblock(wave);
+  const int Cw = C0 + 32 * cbw;
+  const int lim = DIAG ? diag_lim(cbw) : 8;
+  const int ncb = (C + 31) / 32;
+  // fragments: block cb of 32 columns, step k, half q at ((cb * nks + k) * 2 + q) * 256 floats
+  const float* pr = XC + ((int64_t)min(R0 / 32 + wave, ncb - 1) * nks * 128 + lane) * 4;
+  const float* pc = XC + ((int64_t)min(Cw / 32, ncb - 1) * nks * 128 + lane) * 4;
+  constexpr int NB = XBLK<DIAG>;
+  floatx16 acc[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+  const int64_t last = kend - 1;
+#pragma unroll
+  for (int h = 0; h < X32DEPTH - 1; ++h)
+    stage_step32(L.s[h], reinterpret_cast<const uint16_t*>(pr), reinterpret_cast<const uint16_t*>(pr + 256), 1024, pc,
+                 sg, wave, lane, min(kbeg + h, last));
+  XWAIT_VM(4 * (X32DEPTH - 2));         // this wave's staging of step kbeg
+  RQ_STAGE_BARRIER();                   // and the other waves'
+  float w[8];
+  {
+    float x[8], sv[8];
+    read_col32(L.s[0], wave, lane, x, sv);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = x[e] * sv[e];
+  }
+  const int64_t n = kend - kbeg;
+  int64_t k = kbeg;
+  constexpr auto round = std::make_integer_sequence<int, X32DEPTH>();
+  for (; k + X32DEPTH <= kend; k += X32DEPTH)
+    x32_round<DIAG>(w, acc, L, pr, pc, sg, wave, lane, k, last, cbw, lim, X32DEPTH, round);
+  x32_round<DIAG>(w, acc, L, pr, pc, sg, wave, lane, k, last, cbw, lim, (int)(n % X32DEPTH), round);
+  XWAIT_VM(0);
+
+  if (part) {
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (!DIAG || bi < lim) part[(bi * 16 + e) * XTHREADS + tid] = acc[bi][e];
+    return;
+  }
+  const int j = Cw + fr;
+#pragma unroll
+  for (int bi = 0; bi < NB; ++bi) {
+    if (DIAG && bi >= lim) continue;
+    const int rb = diag_rows<DIAG>(cbw, bi);
+    const bool flip = DIAG && rb > cbw;           // below a diagonal tile's diagonal: the transpose
+    const int i0 = R0 + 32 * rb + 4 * fh;
+    float* ph = Hg + (flip ? (int64_t)j * C + i0 : (int64_t)i0 * C + j);
+    const int64_t st = flip ? 1 : C;
+    float hv[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int d = 8 * (e >> 2) + (e & 3);
+      hv[e] = (i0 + d < C && j < C) ? ph[d * st] : 0.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int d = 8 * (e >> 2) + (e & 3);
+      if (i0 + d < C && j < C) ph[d * st] = hv[e] + acc[bi][e];
+    }
+  }
+}
+
+__global__ __launch_bounds__(XTHREADS, 1) void k_hessian_x32(const float* __restrict__ XC, int C,
+                                                             const float* __restrict__ sT, int64_t lds_stride,
+                                                             HTargets tg, int ntarg, int nt, int ntiles, int64_t nks,
+                                                             int64_t nst, int full, TailPlan P,
+                                                             float* __restrict__ ws) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds0[X3_STAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t lds1[X3_STAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t lds2[X3_STAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t lds3[X3_STAGE];
+  static_assert(X32DEPTH == 4, "stage arrays");
+  const XStages L{{lds0, lds1, lds2, lds3}};
+  const int total = ntiles * ntarg;
+  const int b = blockIdx.x;
+  auto tile = [&](int logical, int64_t kbeg, int64_t kend, float* part) __attribute__((always_inline)) {
+    int g, ti, tj;
+    item_tile(logical, ntarg, nt, g, ti, tj);
+    const int R0 = ti * XT, C0 = tj * XT;
+    if (R0 == C0)
+      x32_tile<true>(XC, nks, C, sT + (int64_t)g * lds_stride, tg.H[g], R0, C0, kbeg, kend, part, L);
+    else
+      x32_tile<false>(XC, nks, C, sT + (int64_t)g * lds_stride, tg.H[g], R0, C0, kbeg, kend, part, L);
+  };
+  // (ranges in runs per XCD; the diagonal slices, which may outnumber the free CUs, in turn)
+  const int w = b < full ? -1 : b - full < P.nod ? xcd_run(b - full, P.nod) : b - full;
+  whole_or_tail(tile, b < full ? item_position(b, full, nt * (nt - 1) / 2 * ntarg) : 0, w, P, nst, full, total, ws);
 }
 
 // Pre-pass over one 64-column x 256-token block of X: the block in the fragment-blocked
@@ -1354,8 +1525,8 @@ __global__ __launch_bounds__(256) void k_xfinish(int C, int nchunk, int ntarg, c
   }
 }
 
-// fp32 X, pass 1 over one 64-column x 256-token block: the block as fp32 column fragments for
-// k_hessian_split32 (per 32 columns and 16-token step, 2 KB: half q in {0, 1}, lane
+// fp32 X, pass 1 over one 64-column x 256-token block: the block as fp32 fragments for
+// k_hessian_x32 and k_hessian_split32 (per 32 columns and 16-token step, 2 KB: half q in {0, 1}, lane
 // L = fr + 32 fh holding tokens 8 fh + 4 q .. +3 of column fr; zeros past ntok and C), each
 // column's max |x| and its level-2 act_square sum for this block (as k_xprep), and (first
 // column block only) the targets' saliencies.  LDS holds the block column-major, row stride 257
@@ -1754,7 +1925,7 @@ hipEvent_t timing_begin(hipStream_t s) {
 // Concurrent workgroups of a Hessian kernel on the current device (CUs x occupancy).
 template <typename K>
 int kernel_slots(K kfn, int threads, int which) {
-  static int cache[3][64];
+  static int cache[4][64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   if (cache[which][dev] > 0) return cache[which][dev];
@@ -1893,16 +2064,22 @@ int launch_act_square(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int
 // 16 diagonal items on 256 workgroups), product kernels of a call: every item whole 2.09 ms,
 // ranges 1.61 ms; C = 2048, four fp16 targets (112 + 32 items): 1.62 -> 1.50 ms for the call.
 constexpr int64_t XTAIL_RANGE = 60;
+// k_hessian_x32's steps are four times as long (3.9 us against 1), so its tails are cut finer: C = 4096, one
+// target, 1000 tokens (136 items) 286 us uncut, 225 in ranges; C = 768, one target, 16384 tokens (6 items)
+// 297 us with 16 slices, 197 with 32.
+constexpr int64_t X32TAIL_RANGE = 15, X32TAIL_SLICES = 32;
 
-TailPlan split_tail(int64_t total, int64_t od_items, int64_t nks, int slots, int64_t max_parts) {
+TailPlan split_tail(int64_t total, int64_t od_items, int64_t nks, int slots, int64_t max_parts,
+                    int64_t range = XTAIL_RANGE, int64_t max_slices = 16, int64_t min_tail = 0) {
   TailPlan P{0, 0, 0, 1};
-  if (slots <= 0 || total <= 0 || total % slots == 0) return P;
-  const int tail = (int)(total % slots);
+  if (slots <= 0 || total <= 0) return P;
+  const int tail = (int)(total % slots > min_tail ? total % slots : min_tail);
+  if (tail == 0) return P;
   const int64_t full = total - tail;
   P.od = (int)(od_items > full ? od_items - full : 0);
   P.dg = tail - P.od;
   P.nod = P.od;
-  const int64_t most = nks / 4 < 16 ? nks / 4 : 16;
+  const int64_t most = nks / 4 < max_slices ? nks / 4 : max_slices;
   int64_t S = slots / tail;
   if (S > most) S = most;
   if (S < 1) S = 1;
@@ -1915,7 +2092,7 @@ TailPlan split_tail(int64_t total, int64_t od_items, int64_t nks, int slots, int
   }
   const TailPlan R{P.od, P.dg, (int)(slots - P.dg * S), P.sd};
   if (P.od > 0 && (S < most || full > 0) && R.nod > P.nod && R.slots() <= max_parts &&
-      nks * P.od / R.nod + XTAIL_RANGE < nks / S)
+      nks * P.od / R.nod + range < nks / S)
     return R;
   return P;
 }
@@ -1924,13 +2101,13 @@ struct SplitLayout {
   int64_t ntok_p, nchunk, off_part, off_xt, off_st, off_m, off_a, off_s, off_scale, bytes;
 };
 
-SplitLayout split_layout(int64_t ntok, int C, int ntarg, int64_t parts) {
+SplitLayout split_layout(int64_t ntok, int C, int ntarg, int64_t parts, int xbytes = 2) {
   SplitLayout L;
   L.ntok_p = ((ntok + XTOK - 1) / XTOK) * XTOK;
   L.nchunk = L.ntok_p / XTOK;
   L.off_part = act_off() + act_plan(ntok, C).bytes;
   L.off_xt = L.off_part + align256(parts * (int64_t)XPART * 4);
-  L.off_st = L.off_xt + align256((int64_t)((C + 31) / 32) * 32 * L.ntok_p * 2);
+  L.off_st = L.off_xt + align256((int64_t)((C + 31) / 32) * 32 * L.ntok_p * xbytes);
   L.off_m = L.off_st + align256((int64_t)ntarg * L.ntok_p * 4);
   L.off_a = L.off_m + align256(L.nchunk * C * 4);
   L.off_s = L.off_a + align256(L.nchunk * C * 4);
@@ -2127,17 +2304,99 @@ int launch_split32(const float* x, int64_t ntok, int64_t ldx, int C, const HTarg
   return RQ_OK;
 }
 
+int x32_slots() { return kernel_slots(k_hessian_x32, XTHREADS, 3); }
+
+// k_hessian_x32 has k_xprep32's launch before it and tiles of 256 columns: from 256 tokens, where the
+// tail's slices spread its tiles over the CUs (two slots per tile), and from 512 otherwise.  Whole call,
+// k_hessian_accum -> k_hessian_x32, C x targets: 256 tokens 256 x 1 57 -> 37 us, 1024 x 4 143 -> 66,
+// 2048 x 4 103 -> 110, 4096 x 1 102 -> 101; 128 tokens 33 -> 49 (1024 x 1), 67 -> 111 (2048 x 4);
+// 512 tokens 2048 x 1 202 -> 67, 2048 x 4 151 -> 153, 3072 x 4 279 -> 225, 4096 x 1 153 -> 144; 4096 tokens
+// 256 x 1 95 -> 68, 2048 x 3 595 -> 507, 4096 x 4 2540 -> 2194.
+bool x32_pays(int64_t ntok, int C, int ntarg) {
+  int nt, ntiles;
+  int64_t total;
+  split_items(C, ntarg, &nt, &ntiles, &total);
+  return ntok >= (2 * total <= x32_slots() ? 256 : 512);
+}
+
+// The diagonal items (the last in order, 5/8 of the others' work each) are in the tail, whatever the last
+// round holds, as slices of at most 2048 tokens, 4 or more from 1024 tokens on: short ones level the end
+// of the launch (2 slices of 4096 tokens, C = 4096 x 1: 851 us, 4: 710, 1: 680), and the diagonal's
+// sums, which grow the most, are chains no longer than k_hessian_accum's slices had (C = 3072 x 3, 16384
+// tokens, H's error against 64 bits: 1.05e-6 there, 2.3e-6 with whole chains, 8.3e-7 so).  At most
+// 1024 partial tiles (256 MB) for it.
+constexpr int64_t X32DIAG_STEPS = 128, X32DIAG_SLOTS = 1024;
+
+TailPlan x32_tail(int64_t ntok, int C, int ntarg, int64_t max_parts) {
+  int nt, ntiles;
+  int64_t total;
+  split_items(C, ntarg, &nt, &ntiles, &total);
+  const int64_t dg = (int64_t)nt * ntarg, nst = (ntok + 15) / 16;
+  const int slots = x32_slots();
+  TailPlan P = split_tail(total, total - dg, nst, slots, max_parts, X32TAIL_RANGE, X32TAIL_SLICES,
+                          total > slots ? dg : 0);
+  int64_t sd = (nst + X32DIAG_STEPS - 1) / X32DIAG_STEPS;
+  if (nst > 64 && sd < 4) sd = 4;
+  if (sd > X32DIAG_SLOTS / dg) sd = X32DIAG_SLOTS / dg;
+  if (sd > P.sd && P.dg == dg && P.od_slots() + dg * sd <= max_parts) P.sd = (int)sd;
+  return P;
+}
+
+int64_t x32_ws_need(int64_t ntok, int C, int ntarg) {
+  return split_layout(ntok, C, ntarg, x32_tail(ntok, C, ntarg, INT64_MAX).slots(), 4).bytes;
+}
+
+int launch_x32(const float* x, int64_t ntok, int64_t ldx, int C, const HTargets& tg, int ntarg, void* ws,
+               int64_t ws_bytes, hipStream_t s) {
+  int nt, ntiles;
+  int64_t total;
+  split_items(C, ntarg, &nt, &ntiles, &total);
+  if (total > 0x7fffffff / 8) return RQ_EINVAL;
+  const bool vec_ok = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && (((size_t)ldx * 4) % 16 == 0);
+  SplitLayout L = split_layout(ntok, C, ntarg, 0, 4);
+  const int64_t nst = (ntok + 15) / 16;           // the chunk's last steps hold zeros
+  const TailPlan P = x32_tail(ntok, C, ntarg, (ws_bytes - L.bytes) / ((int64_t)XPART * 4));
+  L = split_layout(ntok, C, ntarg, P.slots(), 4);
+  char* wb = reinterpret_cast<char*>(ws);
+  float* xc = reinterpret_cast<float*>(wb + L.off_xt);
+  float* sT = reinterpret_cast<float*>(wb + L.off_st);
+  float* apart = reinterpret_cast<float*>(wb + L.off_a);
+  hipLaunchKernelGGL(k_xprep32, dim3((C + XPC - 1) / XPC, (unsigned)L.nchunk), dim3(256), 0, s, x, ntok, ldx, C,
+                     vec_ok, reinterpret_cast<float4*>(xc), L.ntok_p / 16, tg, ntarg, sT, L.ntok_p,
+                     reinterpret_cast<float*>(wb + L.off_m), apart, reinterpret_cast<float*>(wb + L.off_s));
+  RQ_CHECK_LAUNCH();
+  {
+    const int rc = launch_act_square(x, RQ_F32, ntok, ldx, C, tg, ntarg, apart, wb + act_off(), s);
+    if (rc) return rc;
+  }
+  const int full = (int)(total - P.items());
+  float* wsf = reinterpret_cast<float*>(wb + L.off_part);
+  hipEvent_t stop = timing_begin(s);
+  hipLaunchKernelGGL(k_hessian_x32, dim3((unsigned)(full + P.wgs())), dim3(XTHREADS), 0, s, xc, C, sT, L.ntok_p, tg,
+                     ntarg, nt, ntiles, L.ntok_p / 16, nst, full, P, wsf);
+  RQ_CHECK_LAUNCH();
+  {
+    const int rc = launch_split_reduce(wsf, P, nst, full, ntarg, nt, C, 1, nullptr, nullptr, tg, s);
+    if (rc) return rc;
+  }
+  if (stop && hipEventRecord(stop, s) != hipSuccess) return RQ_EHIP;
+  return RQ_OK;
+}
+
 int launch_hessian(const void* x, int x_dtype, int64_t ntok, int64_t ldx, int C, const HTargets& tg,
                    int ntarg, void* ws, int64_t ws_bytes, hipStream_t s) {
   const bool aligned = ws && ((reinterpret_cast<uintptr_t>(ws) & 255) == 0);
   if (x_dtype != RQ_F32 && g_hmath.load() != RQ_HMATH_FP32 && aligned &&
       ws_bytes >= split_layout(ntok, C, ntarg, 0).bytes)
     return launch_split(x, x_dtype, ntok, ldx, C, tg, ntarg, ws, ws_bytes, s);
-  // fp32 X: the split kernel (products within ~2^-20.5) only in the opt-in two-piece mode; by
-  // default the fp32 MFMA kernel below forms the reference's products exactly
+  // fp32 X: the split kernel (products within ~2^-20.5) only in the opt-in two-piece mode; else
+  // fp32 MFMAs form the reference's products exactly, k_hessian_x32 where the workspace has room for
+  // the chunk in fragments
   if (x_dtype == RQ_F32 && g_hmath.load() == RQ_HMATH_SPLIT16 && aligned &&
       ws_bytes >= split_layout32(ntok, C, ntarg, 0).bytes)
     return launch_split32(static_cast<const float*>(x), ntok, ldx, C, tg, ntarg, ws, ws_bytes, s);
+  if (x_dtype == RQ_F32 && aligned && x32_pays(ntok, C, ntarg) && ws_bytes >= split_layout(ntok, C, ntarg, 0, 4).bytes)
+    return launch_x32(static_cast<const float*>(x), ntok, ldx, C, tg, ntarg, ws, ws_bytes, s);
   const int nt = (C + HT - 1) / HT;
   const int ntiles = nt * (nt + 1) / 2;
   const int64_t total = (int64_t)ntiles * ntarg;
@@ -2203,6 +2462,8 @@ extern "C" int64_t rq_hessian_workspace_bytes(int64_t ntok, int C, int ntargets,
     int64_t b = hessian_ws_bytes(ntok, C, tail, S);
     const int64_t bs = x_dtype == RQ_F32 ? split32_ws_need(ntok, C, n) : split_ws_need(ntok, C, n);
     if (bs > b) b = bs;
+    const int64_t bx = x_dtype == RQ_F32 && x32_pays(ntok, C, n) ? x32_ws_need(ntok, C, n) : 0;
+    if (bx > b) b = bx;
     if (b > need) need = b;
   }
   return need;

@@ -67,12 +67,12 @@ int64_t rq_hessian_workspace_bytes(int64_t ntok, int C, int ntargets, int x_dtyp
  * RQ_HMATH_SPLIT16X3 (default): the reference's fp32 products exactly.  fp16 and bf16 X with
  *   the weighted operand in three pieces (11 + 11 + 2 or 8 + 8 + 8 bits; for fp16, every
  *   operand within 2^15 of its column's largest, below that within 2^-40 of the largest);
- *   fp32 X on the fp32 MFMA kernel.
+ *   fp32 X on fp32 MFMAs.
  * RQ_HMATH_SPLIT16 (opt-in, faster, narrower products): fp16 X in two pieces (22 of the
  *   operand's 24 bits: each product within 2^-23 relative of the reference's, 2/3 of the MFMA
  *   work), bf16 X in three; fp32 X with x itself in two fp16 pieces, three MFMAs per product
- *   (hi w0, hi w1, lo w0: each product within ~2^-20.5 relative; k_hessian_split32, about 3x
- *   the fp32 MFMA kernel's speed).
+ *   (hi w0, hi w1, lo w0: each product within ~2^-20.5 relative; k_hessian_split32, about 2.4x
+ *   the speed of k_hessian_x32).
  * RQ_HMATH_FP32: fp32 MFMA on converted operands for every input type (exact fp32 products).
  * mode < 0 queries.  Returns the previous mode, or RQ_EINVAL.  No counterpart in the
  * reference (its bmm runs in fp32, gptq_plus_utils.py:845-847). */
@@ -81,7 +81,7 @@ int64_t rq_hessian_workspace_bytes(int64_t ntok, int C, int ntargets, int x_dtyp
 #define RQ_HMATH_SPLIT16X3 2
 int rq_hessian_math(int mode);
 /* Measurement hook, no counterpart in the reference: the next Hessian product-kernel launch
- * (k_hessian_split or k_hessian_accum, whichever runs; k_hessian_split issues one call's
+ * (k_hessian_split, k_hessian_x32 or k_hessian_accum, whichever runs; k_hessian_split issues one call's
  * items as one dispatch per round of whole items, and the pair brackets all of them) records
  * start_event before it and stop_event after it on its stream, so a caller can time that
  * kernel alone (hipEvent_t handles created with timing enabled; both NULL clears).

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 import torch
 
+from gptq_plus_mp_quant_amd import _native as nat
 from gptq_plus_mp_quant_amd import kernels as K
 from tests._util import rel_fro, rng
 
@@ -275,3 +276,41 @@ def test_split_tail_ranges(n, C, G, dtype):
         ref = H0[t].double() + xd.t().contiguous() @ (xd * s[:, t:t + 1].double())
         got, ref = outs[0][0][t].double()[iu[0], iu[1]], ref[iu[0], iu[1]]
         assert float((got - ref).norm() / ref.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("n,C,G,off", [(256, 257, 3, 0),      # 9 items, slices of the diagonal, ragged blocks
+                                       (512, 2048, 4, 0),     # 144 items, whole
+                                       (1025, 513, 2, 1),     # one row past a step and a chunk, x not 16-byte aligned
+                                       (2100, 3072, 2, 0),    # ranges beside more diagonal slices than free slots
+                                       (600, 2048, 15, 0),    # whole items of two rounds, then the diagonal
+                                       (5000, 300, 32, 0)])   # diagonal slices limited by their partial tiles
+def test_fp32_x_fragments(n, C, G, off):
+    """fp32 X at the sizes that run from fragments: against the fp64 sum within 1e-6 (the module's bar:
+    chains of fp32 additions), the same twice, H += on a non-zero H, act_square as from a workspace
+    too small for them (the other kernel), and that kernel's H within the two errors."""
+    g = torch.Generator(device=DEV).manual_seed(n + C)
+    buf = torch.randn(n * C + off, device=DEV, generator=g)
+    x = buf[off:].view(n, C)
+    s = torch.randn((n, G), device=DEV, generator=g).exp_()
+    H0 = torch.randn((G, C, C), device=DEV, generator=g)
+    lib = nat.load()
+
+    def run(need):
+        H, a = H0.clone(), torch.zeros(C, device=DEV)
+        ws = torch.zeros(max(need, 1), dtype=torch.uint8, device=DEV)
+        assert lib.rq_hessian_accum(nat.ptr(x), nat.RQ_F32, n, C, C, nat.ptr(s), G, G, nat.ptr(H),
+                                    nat.ptr(a), nat.ptr(ws), need, nat.stream_of(DEV)) == nat.RQ_OK
+        torch.cuda.synchronize()
+        return H, a
+
+    need = int(lib.rq_hessian_workspace_bytes(n, C, G, nat.dtype_code(x.dtype)))
+    first, again, small = run(need), run(need), run(0)
+    assert torch.equal(first[0], again[0]) and torch.equal(first[1], again[1])
+    assert torch.equal(first[1], small[1])
+    xd = x.double()
+    iu = torch.triu_indices(C, C, device=DEV)
+    for t in range(G):
+        ref = (H0[t].double() + xd.t().contiguous() @ (xd * s[:, t:t + 1].double()))[iu[0], iu[1]]
+        got, old = first[0][t].double()[iu[0], iu[1]], small[0][t].double()[iu[0], iu[1]]
+        assert float((got - ref).norm() / ref.norm()) <= 1e-6
+        assert float((got - old).norm() / ref.norm()) <= 2e-6
