@@ -76,15 +76,19 @@ __global__ __launch_bounds__(256) void k_find_params(const TW* __restrict__ w, i
 //  - x / s with s shared by all elements: y = RN(1 / s), q0 = RN(x y), then one residual step
 //    q0 + y (x - s q0) in two fused operations is the correctly rounded quotient (Markstein)
 //    while nothing underflows; steps outside [2^-60, 2^60] take the IEEE divide.
-//  - |q - x|^norm in 64-bit arithmetic (mse_pow), a quarter of powf's instructions and closer to
-//    the exact power.
+//  - |q - x|^norm in 64-bit arithmetic (mse_pow), a quarter of powf's instructions.  Its last bit is
+//    not powf's, so it settles only what it can: candidates whose error lies within the two sums'
+//    rounding of the least are summed again with powf (and the IEEE divide), and those sums decide,
+//    so the choice is the one that powf throughout makes.  The candidates in question are kept in
+//    a list as they come (8 for each of a batch's places, a lane each); a wave whose list ran over
+//    goes through its batches again.
 //  - One wave per candidate batch: a lane holds 4 of 256 interleaved partial sums, and 8
 //    candidates are reduced together by halving exchanges (10 shuffles instead of 48), with no
 //    barrier.  Up to MSE_WIDE elements a wave owns one (row, group); wider rows share a
 //    workgroup's 4 waves, which take every fourth batch.
 // 1024 x 4096 fp32 against one 256-thread workgroup per (row, group), every candidate, the IEEE
-// divide and powf: symmetric 16.3 -> 0.43 ms (128-column groups) and 10.7 -> 0.34 ms (per row),
-// asymmetric 16.5 -> 4.2 and 10.5 -> 3.0 ms.
+// divide and powf: symmetric 16.3 -> 0.40 ms (128-column groups) and 10.7 -> 0.34 ms (per row),
+// asymmetric 16.5 -> 4.1 and 10.5 -> 3.1 ms (of which the sums by powf 3 to 5 %).
 constexpr int MSE_WIDE = 1024;          // above: one (row, group) per workgroup
 constexpr int MSE_LDS_MAX = 16384;      // elements staged in LDS; wider groups are read in place
 constexpr int MSE_B = 8;                // candidates per batch
@@ -95,8 +99,9 @@ struct MseLog {
 
 // |d|^p for d >= 0 finite and p > 0, in 64 bits and rounded once: log2(d) = e + log2(c) +
 // log2(m / c) with m / c - 1 within 0.0304 of 0 (a table of 16 centres c), 2^y by its
-// fractional part; both polynomials are near-minimax (2^-36 and 2^-34), so the result is within
-// 0.5 + 2^-9 units of the last place (powf: 1).
+// fractional part.  Both polynomials were fitted for this kernel at Chebyshev nodes of their
+// intervals (errors 2^-36 and 2^-34), so the result is within 0.5 + 2^-10 + p 2^-12 units of
+// the last place (powf: 1).
 __device__ __forceinline__ float mse_pow(float d, double p, const MseLog* tab) {
   const float m = __builtin_amdgcn_frexp_mantf(d);
   const int e = __builtin_amdgcn_frexp_expf(d);
@@ -139,7 +144,8 @@ struct MseGrid {
       const float other = c < steps ? rq_nan_min(hi(0), hi(steps - 1)) : lo(steps - 1);
       *s = rq_clamp_min(m, 1e-5f) / maxq;
       *z = 0.0f;
-      return c < n && !(other > m);
+      // (both sides shrunk alike to one value: the row's)
+      return c < n && !(other > m) && !(c >= steps && lo(k) == m);
     }
     const float xmin1 = fac(c / steps) * xmin, xmax1 = fac(c % steps) * xmax;
     *s = (xmax1 - xmin1) / maxq;
@@ -226,7 +232,7 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
                                                          float* __restrict__ zero) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ MseLog tab[16];
-  __shared__ float best_e[4];
+  __shared__ float best_e[4], best_e2[4];
   __shared__ int best_c[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid < 16) {
@@ -280,91 +286,158 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
   g.sym = SYM;
   g.grid = grid;
   g.steps = steps;
-  g.n = SYM ? 2 * steps : steps * steps;
+  g.n = !live ? 0 : SYM ? 2 * steps : steps * steps;
+  // one step only, the start's (its lower bound), or no error at all: the first candidate wins
+  if (SYM && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
+  if (!SYM && rmin == 0.0f && rmax == 0.0f) g.n = min(g.n, 1);
   const double p = (double)norm;
+  const bool fast = norm > 0.0f && norm < 64.0f;
   // the lane's own candidate among the batch's: bit 5, 4, 3 of the lane
   const int mine = ((lane >> 5) & 1) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1);
-  float be = __builtin_inff();
+  // The least error and its candidate, and the next least: of the 8 lanes that share `mine`, then
+  // of all.
+  float be = __builtin_inff(), be2 = __builtin_inff();
   int bc = -1;
-  for (int b = shared ? wave : 0; b * MSE_B < g.n; b += shared ? 4 : 1) {
-    // lane k < 8 works out candidate k's step; every lane then reads all eight
-    float cs, cz;
-    const bool ok = g.params(b * MSE_B + (lane & (MSE_B - 1)), &cs, &cz);
-    const float cy = 1.0f / cs;
-    // steps for which the residual divide is exact, and finite data (an infinity or NaN in the
-    // row makes every step one)
-    const bool good = cs >= 0x1p-60f && cs <= 0x1p60f && norm > 0.0f && norm < 64.0f;
-    float s[MSE_B], z[MSE_B], y[MSE_B], part[MSE_B];
-#pragma unroll
-    for (int k = 0; k < MSE_B; ++k) {
-      s[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
-      z[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
-      y[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cy), k));
-    }
-    const uint64_t valid = __ballot(ok) & 255, exact = __ballot(good || !ok) & 255;
-    if (!valid) continue;
-    if (exact == 255) {
-      if (STAGED) mse_batch<SYM>(xw, n, lane, s, z, y, maxq, p, tab, part);
-      else mse_batch<SYM>(row, n, lane, s, z, y, maxq, p, tab, part);
-    } else {
-      for (int k = 0; k < MSE_B; ++k) {
-        const float sk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
-        const float zk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
-        const float v = STAGED ? mse_any<SYM>(xw, n, lane, sk, zk, maxq, norm)
-                               : mse_any<SYM>(row, n, lane, sk, zk, maxq, norm);
-#pragma unroll
-        for (int j = 0; j < MSE_B; ++j)
-          if (j == k) part[j] = v;
-      }
-    }
-    // the tree of 64 partial sums (l + (l + 32), + 16, ...), halving the candidates a lane keeps
-    // for the first three levels; each lane ends with the sum of candidate `mine`
-    float h4[4], h2[2];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool up = lane & 32;
-      const float keep = up ? part[k + 4] : part[k], send = up ? part[k] : part[k + 4];
-      h4[k] = keep + __shfl_xor(send, 32, 64);
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const bool up = lane & 16;
-      const float keep = up ? h4[k + 2] : h4[k], send = up ? h4[k] : h4[k + 2];
-      h2[k] = keep + __shfl_xor(send, 16, 64);
-    }
-    const bool up = lane & 8;
-    float err = (up ? h2[1] : h2[0]) + __shfl_xor(up ? h2[0] : h2[1], 8, 64);
-    err += __shfl_xor(err, 4, 64);
-    err += __shfl_xor(err, 2, 64);
-    err += __shfl_xor(err, 1, 64);
-    const int c = b * MSE_B + mine;
-    if ((valid >> mine) & 1) {
-      if (err < be || (err == be && bc >= 0 && g.first(c) < g.first(bc))) {
-        be = err;
-        bc = c;
-      }
-    }
-  }
-  auto merge = [&](float oe, int oc) {
-    if (oc >= 0 && (bc < 0 || oe < be || (oe == be && oc != bc && g.first(oc) < g.first(bc)))) {
-      be = oe;
-      bc = oc;
-    }
+  auto take = [&](float e, int c) {
+    const bool less = e < be || (e == be && bc >= 0 && g.first(c) < g.first(bc));
+    const float other = less ? be : e;
+    be2 = other < be2 ? other : be2;
+    be = less ? e : be;
+    bc = less ? c : bc;
   };
+  // Errors within near(least) of each other are in question: n terms that differ by 2 units of
+  // the last place at most (a unit is 2^-23; and 2 subnormal ones), in sums of n / 256 + 9
+  // roundings each.  near - 1 is over twice the sums' largest relative difference.
+  const float slack = (float)((n + 255) / 256 + 16) * 0x1p-21f, least_e = (float)n * 0x1p-147f;
+  auto near = [&](float e) { return e + e * slack + least_e; };
+  // the list: lane q of the 8 holds entry q
+  float list_e = 0.0f;
+  int list_c = 0, listed = 0;
+  auto all_lanes = [&](float v) {
 #pragma unroll
-  for (int o = 32; o >= 8; o >>= 1) {
-    const float oe = __shfl_xor(be, o, 64);
-    const int oc = __shfl_xor(bc, o, 64);
-    merge(oe, oc);
-  }
-  if (shared) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  };
+  auto merge = [&](float oe, int oc, float oe2) {
+    if (oc >= 0) take(oe, oc);
+    be2 = oe2 < be2 ? oe2 : be2;
+  };
+  auto merge_waves = [&]() {
+    if (!shared) return;
     if (lane == 0) {
       best_e[wave] = be;
+      best_e2[wave] = be2;
       best_c[wave] = bc;
     }
     __syncthreads();
-    for (int k = 0; k < 4; ++k) merge(best_e[k], best_c[k]);
+    be = best_e[0];
+    be2 = best_e2[0];
+    bc = best_c[0];
+    for (int k = 1; k < 4; ++k) merge(best_e[k], best_c[k], best_e2[k]);
+    __syncthreads();
+  };
+  // a candidate by powf: the lane's part of the sum
+  auto any = [&](float sk, float zk) {
+    return STAGED ? mse_any<SYM>(xw, n, lane, sk, zk, maxq, norm) : mse_any<SYM>(row, n, lane, sk, zk, maxq, norm);
+  };
+  // the candidates c of the lanes in `todo`
+  auto evaluate = [&](uint64_t todo, int c) {
+    for (; todo; todo &= todo - 1) {
+      const int l = __builtin_ctzll(todo), cl = __builtin_amdgcn_readlane(c, l);
+      if (be == 0.0f && bc >= 0 && g.first(cl) > g.first(bc)) continue;      // not less than nothing
+      float sk, zk;
+      g.params(cl, &sk, &zk);
+      take(all_lanes(any(sk, zk)), cl);
+    }
+  };
+  bool settled = false;
+  // Pass 0: every candidate, by mse_pow.  Pass 1 (a list that ran over): those in question, by powf.
+  float limit = 0.0f;
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int b = shared ? wave : 0; b * MSE_B < g.n; b += shared ? 4 : 1) {
+      // lane k < 8 works out candidate k's step; every lane then reads all eight
+      float cs, cz;
+      const bool ok = g.params(b * MSE_B + (lane & (MSE_B - 1)), &cs, &cz);
+      const float cy = 1.0f / cs;
+      // steps for which the residual divide is exact, and finite data (an infinity or NaN in the
+      // row makes every step one)
+      const bool good = fast && cs >= 0x1p-60f && cs <= 0x1p60f;
+      float s[MSE_B], z[MSE_B], y[MSE_B], part[MSE_B];
+#pragma unroll
+      for (int k = 0; k < MSE_B; ++k) {
+        s[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
+        z[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
+        y[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cy), k));
+      }
+      const uint64_t valid = __ballot(ok) & 255, exact = __ballot(good || !ok) & 255;
+      if (!valid) continue;
+      if (exact == 255) {
+        if (STAGED) mse_batch<SYM>(xw, n, lane, s, z, y, maxq, p, tab, part);
+        else mse_batch<SYM>(row, n, lane, s, z, y, maxq, p, tab, part);
+      } else {
+        for (int k = 0; k < MSE_B; ++k) {
+          const float sk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cs), k));
+          const float zk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cz), k));
+          const float v = any(sk, zk);
+#pragma unroll
+          for (int j = 0; j < MSE_B; ++j)
+            if (j == k) part[j] = v;
+        }
+      }
+      // the tree of 64 partial sums (l + (l + 32), + 16, ...), halving the candidates a lane keeps
+      // for the first three levels; each lane ends with the sum of candidate `mine`
+      float h4[4], h2[2];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool up = lane & 32;
+        const float keep = up ? part[k + 4] : part[k], send = up ? part[k] : part[k + 4];
+        h4[k] = keep + __shfl_xor(send, 32, 64);
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const bool up = lane & 16;
+        const float keep = up ? h4[k + 2] : h4[k], send = up ? h4[k] : h4[k + 2];
+        h2[k] = keep + __shfl_xor(send, 16, 64);
+      }
+      const bool up = lane & 8;
+      float err = (up ? h2[1] : h2[0]) + __shfl_xor(up ? h2[0] : h2[1], 8, 64);
+      err += __shfl_xor(err, 4, 64);
+      err += __shfl_xor(err, 2, 64);
+      err += __shfl_xor(err, 1, 64);
+      const bool there = (valid >> mine) & 1;
+      const int c = b * MSE_B + mine;
+      if (pass == 0) {
+        if (there && err <= near(be)) {
+          if (be > near(err)) listed = 0;
+          if ((lane & 7) == listed) {
+            list_e = err;
+            list_c = c;
+          }
+          ++listed;
+        }
+        if (there) take(err, c);
+      } else {
+        evaluate(__ballot(there && err <= limit && (lane & 7) == 0), c);
+      }
+    }
+    if (pass == 1) break;
+#pragma unroll
+    for (int o = 32; o >= 8; o >>= 1) {
+      const float oe = __shfl_xor(be, o, 64), oe2 = __shfl_xor(be2, o, 64);
+      const int oc = __shfl_xor(bc, o, 64);
+      merge(oe, oc, oe2);
+    }
+    merge_waves();
+    limit = near(be);
+    settled = !fast || be2 > limit;                     // (the same in all waves of a (row, group))
+    if (settled) break;
+    be = be2 = __builtin_inff();
+    bc = -1;
+    if (__ballot(listed > 8)) continue;
+    evaluate(__ballot((lane & 7) < listed && list_e <= limit), list_c);
+    break;
   }
+  if (!settled) merge_waves();
   if (live && lane == 0 && (!shared || wave == 0)) {
     float bs, bz;
     if (bc >= 0) g.params(bc, &bs, &bz);

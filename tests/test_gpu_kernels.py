@@ -827,6 +827,80 @@ def test_find_params_mse_widths(n, gs, sym):
             assert abs(e_gpu - e_ora) <= 2.0 ** -13 * e_ora, (i, e_gpu, e_ora)
 
 
+def _search32(W, maxq, sym, clip_zero, norm=2.4, grid=50, maxshrink=0.5):
+    """The clip search in 32 bits as find_params defines it, op by op on the GPU: every (i, j) of the
+    grid in order, the error as 256 interleaved partial sums of powf terms added by halves, the first
+    strict minimum (rows without NaN)."""
+    R, n = W.shape
+    x = W.float()
+    lo, hi = x.amin(1), x.amax(1)
+    scale, zero = K.find_params(W, maxq, sym, clip_zero=clip_zero)
+    scale, zero = scale[0].clone(), zero[0].clone()
+    if clip_zero:
+        lo, hi = lo.clamp(max=0.0), hi.clamp(min=0.0)
+    if not sym:
+        none = (lo == 0) & (hi == 0)
+        lo, hi = torch.where(none, -1.0, lo), torch.where(none, 1.0, hi)
+    best = torch.full((R,), float("inf"), device=W.device)
+    steps = int(maxshrink * grid)
+    top = torch.full((1,), float(maxq), device=W.device)      # (a Python divisor would be inverted first)
+    for i in range(steps):
+        for j in range(steps):
+            l1, h1 = (1 - i / grid) * lo, (1 - j / grid) * hi
+            if sym:
+                s = torch.maximum(l1.abs(), h1).clamp(min=1e-5) / top
+                z = torch.zeros_like(s)
+                q = s[:, None] * torch.clamp(torch.round(x / s[:, None]), -(maxq + 1), maxq)
+            else:
+                s = (h1 - l1) / top
+                z = torch.round(-l1 / s)
+                q = s[:, None] * (torch.clamp(torch.round(x / s[:, None]) + z[:, None], 0, maxq) - z[:, None])
+            e = torch.nn.functional.pad((q - x).abs().pow(norm), (0, -n % 256))
+            p = torch.zeros((R, 256), device=W.device)
+            for c in range(0, e.shape[1], 256):
+                p = p + e[:, c:c + 256]
+            while p.shape[1] > 1:
+                h = p.shape[1] // 2
+                p = p[:, :h] + p[:, h:]
+            better = p[:, 0] < best
+            best = torch.where(better, p[:, 0], best)
+            scale, zero = torch.where(better, s, scale), torch.where(better, z, zero)
+    return scale, zero
+
+
+@pytest.mark.parametrize("R,n,sym,clip_zero,kw", [
+    (40000, 128, True, True, {}), (20000, 128, False, True, {}), (20000, 64, False, False, {}),
+    (3000, 1000, False, True, {}), (300, 1000, False, True, {}), (100, 5000, True, True, {}),
+    (10, 17000, True, False, {}),
+    (5000, 100, True, True, {"norm": 2.0}), (5000, 100, False, True, {"norm": 1.3}),
+    (2000, 100, True, True, {"norm": 30.0}), (500, 100, True, True, {"norm": 70.0})])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_find_params_mse_choice(R, n, sym, clip_zero, kw, dtype):
+    """The search takes the candidate that its 32-bit definition takes, near ties included (no
+    tolerance): scales and zeros bit for bit, for rows of equal and of one-signed values, zeros,
+    rows so small that powers underflow and rows near 1e15 whose powers overflow."""
+    g = torch.Generator(device=DEV).manual_seed(R + n)
+    W = torch.randn((R, n), device=DEV, generator=g) * 0.02
+    W[::50] = 0
+    W[1::50] = W[1::50].abs()
+    W[2::50] = -W[2::50].abs() - 0.01
+    W[3::50] = 0.25
+    W[4::50, ::2] = -W[4::50, :n - n // 2].abs()
+    for k, f in enumerate((1e-5, 1e-16, 1e-17, 1e-18, 1e-20, 1e-28, 1e-36, 1e15, 1e17, 1e25)):
+        W[5 + k::50] *= f
+    W[15::50, 0] = W[15::50].abs().amax(1)
+    W[15::50, n - 1] = -W[15::50, 0]                          # the two ends equal
+    W = W.to(dtype)
+    q = make_quantizer(4, sym, mse=True)
+    for name, v in kw.items():
+        setattr(q, name, v)
+    scale, zero = K.find_params_mse(W, int(q.maxq), sym, clip_zero=clip_zero, **kw)
+    es, ez = _search32(W, int(q.maxq), sym, clip_zero, **kw)
+    # (a zero of either sign)
+    bad = torch.nonzero((scale[0].view(torch.int32) != es.view(torch.int32)) | (zero[0] != ez)).flatten()
+    assert bad.numel() == 0, (bad[:8].tolist(), scale[0][bad[:8]].tolist(), es[bad[:8]].tolist())
+
+
 @pytest.mark.parametrize("case", ["plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "inf_w", "nan_w", "big_w"])
 @pytest.mark.parametrize("count", [128, 100, 17])
 @pytest.mark.parametrize("atomic", [False, True])
