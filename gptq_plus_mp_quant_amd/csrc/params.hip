@@ -72,7 +72,8 @@ __global__ __launch_bounds__(256) void k_find_params(const TW* __restrict__ w, i
 // Bound by VALU issue: a candidate costs every element a divide, a round, a clamp and a power.
 //  - Symmetric: s depends on (i, j) only through max(|xmin1|, xmax1), one of 2 * steps values, and
 //    equal steps have equal errors, so 2 * steps candidates are evaluated instead of steps^2
-//    (50 instead of 625 at the default grid).
+//    (50 instead of 625 at the default grid).  Shrunk past zero (maxshrink > 1) the factors
+//    change sign and |xmin1| no longer falls with i: there all steps^2 are evaluated.
 //  - x / s with s shared by all elements: y = RN(1 / s), q0 = RN(x y), then one residual step
 //    q0 + y (x - s q0) in two fused operations is the correctly rounded quotient (Markstein)
 //    while nothing underflows; steps outside [2^-60, 2^60] take the IEEE divide.
@@ -127,17 +128,19 @@ __device__ __forceinline__ float mse_pow(float d, double p, const MseLog* tab) {
   return d == 0.0f ? 0.0f : v;
 }
 
-// The step and zero of candidate c, and whether it is one of the grid's.  Symmetric candidates:
-// c < steps is |xmin| shrunk by row c of the grid (where some column leaves xmax no larger), the
-// others xmax shrunk by column c - steps.
+// The step and zero of candidate c, and whether it is one of the grid's.  Distinct steps of a
+// symmetric grid (`distinct`, factors that fall from 1 and stay non-negative): c < steps is |xmin|
+// shrunk by row c of the grid (where some column leaves xmax no larger), the others xmax shrunk by
+// column c - steps.  Else candidate c is row c / steps, column c % steps.
 struct MseGrid {
   float xmin, xmax, maxq;
   int sym, grid, steps, n;
+  bool distinct;
   __device__ __forceinline__ float fac(int i) const { return (float)(1.0 - (double)i / (double)grid); }
   __device__ __forceinline__ float lo(int i) const { return fabsf(fac(i) * xmin); }
   __device__ __forceinline__ float hi(int j) const { return fac(j) * xmax; }
   __device__ __forceinline__ bool params(int c, float* s, float* z) const {
-    if (sym) {
+    if (distinct) {
       const int k = c < steps ? c : c - steps;
       const float m = c < steps ? lo(k) : hi(k);
       // the other side's smallest value decides whether max() ever takes m
@@ -148,13 +151,18 @@ struct MseGrid {
       return c < n && !(other > m) && !(c >= steps && lo(k) == m);
     }
     const float xmin1 = fac(c / steps) * xmin, xmax1 = fac(c % steps) * xmax;
+    if (sym) {
+      *s = rq_clamp_min(rq_nan_max(fabsf(xmin1), xmax1), 1e-5f) / maxq;
+      *z = 0.0f;
+      return c < n;
+    }
     *s = (xmax1 - xmin1) / maxq;
     *z = __builtin_rintf(-xmin1 / *s);
     return c < n;
   }
   // place of candidate c in the search order (row by row), for equal errors
   __device__ int first(int c) const {
-    if (!sym) return c;
+    if (!distinct) return c;
     const bool row = c < steps;
     const int k = row ? c : c - steps;
     const float m = row ? lo(k) : hi(k);
@@ -286,9 +294,10 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
   g.sym = SYM;
   g.grid = grid;
   g.steps = steps;
-  g.n = !live ? 0 : SYM ? 2 * steps : steps * steps;
+  g.distinct = SYM && steps - 1 <= grid;
+  g.n = !live ? 0 : g.distinct ? 2 * steps : steps * steps;
   // one step only, the start's (its lower bound), or no error at all: the first candidate wins
-  if (SYM && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
+  if (g.distinct && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
   if (!SYM && rmin == 0.0f && rmax == 0.0f) g.n = min(g.n, 1);
   const double p = (double)norm;
   const bool fast = norm > 0.0f && norm < 64.0f;

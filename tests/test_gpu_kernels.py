@@ -901,6 +901,26 @@ def test_find_params_mse_choice(R, n, sym, clip_zero, kw, dtype):
     assert bad.numel() == 0, (bad[:8].tolist(), scale[0][bad[:8]].tolist(), es[bad[:8]].tolist())
 
 
+@pytest.mark.parametrize("sym,kw", [
+    (True, {"maxshrink": 1.2, "grid": 10}), (True, {"maxshrink": 1.5}), (True, {"maxshrink": 2.6, "grid": 10}),
+    (True, {"maxshrink": 1.0, "grid": 10}), (True, {"maxshrink": 1.1, "grid": 10}), (False, {"maxshrink": 1.5, "grid": 10})])
+@pytest.mark.parametrize("n,clip_zero", [(100, True), (1100, False)])
+def test_find_params_mse_past_zero(sym, kw, n, clip_zero):
+    """maxshrink above 1: the factors 1 - i / grid change sign, so |xmin| shrunk no longer falls row by
+    row (and above 2 it outgrows the row's).  A low norm and outliers at either end draw the choice to
+    small steps; scale and zero are those of the whole grid, bit for bit."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    W = torch.randn((1000, n), device=DEV, generator=g) * 0.02
+    for k, f in enumerate((-3.0, -8.0, -20.0, -60.0, 8.0, 60.0)):
+        W[k::7, 0] = f * W[k::7].abs().amax(1)
+    W[6::49] *= 1e-5
+    for norm in (0.6, 2.4):
+        scale, zero = K.find_params_mse(W, 7 if sym else 15, sym, clip_zero=clip_zero, norm=norm, **kw)
+        es, ez = _search32(W, 7 if sym else 15, sym, clip_zero, norm, **kw)
+        bad = torch.nonzero((scale[0].view(torch.int32) != es.view(torch.int32)) | (zero[0] != ez)).flatten()
+        assert bad.numel() == 0, (bad.numel(), bad[:4].tolist(), scale[0][bad[:4]].tolist(), es[bad[:4]].tolist())
+
+
 @pytest.mark.parametrize("case", ["plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "inf_w", "nan_w", "big_w"])
 @pytest.mark.parametrize("count", [128, 100, 17])
 @pytest.mark.parametrize("atomic", [False, True])
