@@ -128,6 +128,9 @@ __device__ __forceinline__ float mse_pow(float d, double p, const MseLog* tab) {
   return d == 0.0f ? 0.0f : v;
 }
 
+// No factor 1 - i / grid below zero.
+__host__ __device__ constexpr bool mse_distinct(int grid, int steps) { return steps - 1 <= grid; }
+
 // The step and zero of candidate c, and whether it is one of the grid's.  Distinct steps of a
 // symmetric grid (`distinct`, factors that fall from 1 and stay non-negative): c < steps is |xmin|
 // shrunk by row c of the grid (where some column leaves xmax no larger), the others xmax shrunk by
@@ -161,14 +164,14 @@ struct MseGrid {
     return c < n;
   }
   // place of candidate c in the search order (row by row), for equal errors
-  __device__ int first(int c) const {
+  __device__ int64_t first(int c) const {
     if (!distinct) return c;
     const bool row = c < steps;
     const int k = row ? c : c - steps;
     const float m = row ? lo(k) : hi(k);
     int o = 0;
     while (o < steps - 1 && (row ? hi(o) : lo(o)) > m) ++o;
-    return row ? k * steps + o : o * steps + k;
+    return row ? (int64_t)k * steps + o : (int64_t)o * steps + k;
   }
 };
 
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
   g.sym = SYM;
   g.grid = grid;
   g.steps = steps;
-  g.distinct = SYM && steps - 1 <= grid;
+  g.distinct = SYM && mse_distinct(grid, steps);
   g.n = !live ? 0 : g.distinct ? 2 * steps : steps * steps;
   // one step only, the start's (its lower bound), or no error at all: the first candidate wins
   if (g.distinct && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
@@ -788,7 +791,8 @@ int launch_find_params_mse(const TW* w, int R, int C, int64_t ldw, int gs, int n
   const int width = gs < C ? gs : C;
   const int per_wg = width <= MSE_WIDE ? 4 : 1;
   const int64_t items = (int64_t)R * ng, wgs = (items + per_wg - 1) / per_wg;
-  if (wgs > 0x7fffffff || (int64_t)steps * steps > (1 << 28)) return RQ_EINVAL;
+  // candidates are counted in 32 bits (46340^2 < 2^31)
+  if (wgs > 0x7fffffff || steps > (sym && mse_distinct(grid, steps) ? 1 << 29 : 46340)) return RQ_EINVAL;
   const bool staged = width <= MSE_LDS_MAX;
   const size_t lds = staged ? (size_t)per_wg * width * sizeof(float) : 0;
   auto go = [&](auto kernel) {

@@ -921,6 +921,24 @@ def test_find_params_mse_past_zero(sym, kw, n, clip_zero):
         assert bad.numel() == 0, (bad.numel(), bad[:4].tolist(), scale[0][bad[:4]].tolist(), es[bad[:4]].tolist())
 
 
+def test_find_params_mse_fine_grid():
+    """A grid of over 2^28 pairs, symmetric: the choice is as good as that of all its distinct steps in
+    64 bits (sums of 48 terms and a power in 32 bits: within 2^-13 as in the test of widths)."""
+    W = torch.from_numpy(rng(9).standard_normal((4, 48)).astype(np.float32) * 0.02)
+    grid = 40000
+    scale, zero = K.find_params_mse(W.to(DEV), 7, True, grid=grid, maxshrink=0.5)
+    fac = (1 - torch.arange(grid // 2, dtype=torch.float64) / grid).float()
+    for r in range(4):
+        lo, hi = (fac * W[r].min()).abs(), fac * W[r].max()
+        lo, hi = lo[lo >= hi.min()], hi[hi >= lo.min()]
+        steps = torch.cat([lo, hi, scale[0, r].cpu().reshape(1) * 7]) / 7
+        x = W[r].double()[None]
+        s = steps.double()[:, None]
+        e = ((s * torch.clamp(torch.round(x / s), -8, 7) - x).abs() ** 2.4).sum(1)
+        assert float(zero[0, r]) == 0 and float(scale[0, r]) in steps[:-1].tolist()
+        assert float(e[-1]) <= (1 + 2.0 ** -13) * float(e.min())
+
+
 @pytest.mark.parametrize("case", ["plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "inf_w", "nan_w", "big_w"])
 @pytest.mark.parametrize("count", [128, 100, 17])
 @pytest.mark.parametrize("atomic", [False, True])
