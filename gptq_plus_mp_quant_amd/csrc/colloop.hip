@@ -19,12 +19,12 @@
 // rows), so both divides are residual divides: with y = RN(1 / d), made before the loop,
 // q0 = RN(n y) and q0 + y (n - d q0) in two fused operations is the correctly rounded n / d
 // (Markstein) unless something underflows or is not finite.  Steps and diagonals outside
-// [2^-60, 2^60], a non-zero numerator below 2^-70 and non-finite results are noticed (three
-// operations per column beside the chain), and the wave then runs its block again with the IEEE
-// divide (a rolled loop).  No branch is left between columns (a block's missing columns are run as
-// zeros with a unit diagonal), so a column's update overlaps the next one's chain.  A 128-column
-// block alone, against the IEEE divides: 24.7 -> 18.1 us at 1024 rows, 30.4 -> 23.8 us at 4096 rows
-// with the first-order terms.
+// [2^-60, 2^55], a non-zero numerator below 2^-70 (so a quotient below 2^-125, the normal numbers'
+// end) and non-finite results are noticed (three operations per column beside the chain), and the
+// wave then runs its block again with the IEEE divide (a rolled loop).  No branch is left between
+// columns (a block's missing columns are run as zeros with a unit diagonal), so a column's update
+// overlaps the next one's chain.  A 128-column block alone, against the IEEE divides: 24.7 -> 18.1 us
+// at 1024 rows, 30.4 -> 23.8 us at 4096 rows with the first-order terms.
 // The atomic variant (:1238-1288) quantises the block start at once and solves
 // Err * Hinv1 = W - Q - GHinv1 by forward substitution with the same row layout.
 //
@@ -134,7 +134,7 @@ __device__ __forceinline__ float residual_div(float n, float d, float y) {
   const float q0 = n * y;
   return __builtin_fmaf(__builtin_fmaf(-d, q0, n), y, q0);
 }
-__device__ __forceinline__ bool residual_ok(float d) { return fabsf(d) >= 0x1p-60f && fabsf(d) <= 0x1p60f; }
+__device__ __forceinline__ bool residual_ok(float d) { return fabsf(d) >= 0x1p-60f && fabsf(d) <= 0x1p55f; }
 
 // GM: 0 frozen, 1 surrogate_block, 2 surrogate_online, 3 frozen with every in-block update
 // scaled by second_order_scale (block_gd, :1344-1349).  NS register slots per lane: lane t of
