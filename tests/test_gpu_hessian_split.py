@@ -307,6 +307,7 @@ def test_fp32_x_fragments(n, C, G, off):
     first, again, small = run(need), run(need), run(0)
     assert torch.equal(first[0], again[0]) and torch.equal(first[1], again[1])
     assert torch.equal(first[1], small[1])
+    assert not torch.equal(first[0], small[0])        # (the kernels add a sum's terms in different orders)
     xd = x.double()
     iu = torch.triu_indices(C, C, device=DEV)
     for t in range(G):
@@ -314,3 +315,26 @@ def test_fp32_x_fragments(n, C, G, off):
         got, old = first[0][t].double()[iu[0], iu[1]], small[0][t].double()[iu[0], iu[1]]
         assert float((got - ref).norm() / ref.norm()) <= 1e-6
         assert float((got - old).norm() / ref.norm()) <= 2e-6
+
+
+@pytest.mark.parametrize("n,G,frags", [(255, 21, False), (256, 21, True),      # 126 tiles, at most half the slots
+                                       (511, 22, False), (512, 22, True)])     # 132 tiles, more than half
+def test_fp32_x_fragments_from(n, G, frags):
+    """The token counts from which fp32 X runs from fragments: below them a call with a workspace gives
+    the bits of a call without (the other kernel; its 441 or 462 tiles run whole in both), from them on
+    other bits, as its sums have another order."""
+    C = 768
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn((n, C), device=DEV, generator=g)
+    s = torch.randn((n, G), device=DEV, generator=g).exp_()
+    lib = nat.load()
+    got = []
+    for need in (int(lib.rq_hessian_workspace_bytes(n, C, G, nat.dtype_code(x.dtype))), 0):
+        H, a = torch.zeros((G, C, C), device=DEV), torch.zeros(C, device=DEV)
+        ws = torch.zeros(max(need, 1), dtype=torch.uint8, device=DEV)
+        assert lib.rq_hessian_accum(nat.ptr(x), nat.RQ_F32, n, C, C, nat.ptr(s), G, G, nat.ptr(H), nat.ptr(a),
+                                    nat.ptr(ws), need, nat.stream_of(DEV)) == nat.RQ_OK
+        torch.cuda.synchronize()
+        got.append((H, a))
+    assert torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][0], got[1][0]) != frags
