@@ -939,17 +939,17 @@ def test_find_params_mse_fine_grid():
         assert float(e[-1]) <= (1 + 2.0 ** -13) * float(e.min())
 
 
-@pytest.mark.parametrize("case", ["plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "big_diag", "inf_w", "nan_w",
-                                  "big_w"])
+# (the solve's order of NaN and infinity is not pinned, and diagonals of 1e-20 overflow it: not atomic)
+@pytest.mark.parametrize("atomic,case", [
+    (atomic, case) for atomic in (False, True)
+    for case in ("plain", "tiny_w", "tiny_scale", "wide_scale", "small_diag", "big_diag", "inf_w", "nan_w", "big_w")
+    if not (atomic and case in ("inf_w", "nan_w", "small_diag"))])
 @pytest.mark.parametrize("count", [128, 100, 17])
-@pytest.mark.parametrize("atomic", [False, True])
 def test_quant_block_divides(case, count, atomic):
     """The column loop's residual divides and the IEEE divide it falls back to: codes and errors equal
     the reference's operations in fp32, one rounding each (no tolerance), for weights, steps and
     diagonals in and out of the residual divide's range and for blocks narrower than the kernel's.
     (Zeros of either sign are equal.)"""
-    if atomic and case in ("inf_w", "nan_w", "small_diag"):
-        pytest.skip("the solve's order of NaN and infinity is not pinned (diagonals of 1e-20 overflow it)")
     r = rng(count + len(case))
     R, C = 40, count
     W = torch.from_numpy(r.standard_normal((R, C)).astype(np.float32) * 0.02)
@@ -1016,20 +1016,106 @@ def test_quant_block_divides(case, count, atomic):
         assert torch.equal(e_got.nan_to_num(123.0), errs.nan_to_num(123.0))
 
 
+# A step of 2^70 and more takes a wave's rows (4 at a time) through the IEEE divides, and scaling a
+# row with its steps by a power of two scales its errors and leaves its codes.
+WIDE, WIDE_ROWS = 2.0 ** 70, [3, 18, 33]
+
+
+def _grid_steps(qmode, W, C, r):
+    """(scale, col_group) for a mode: per row, or a table of 64-column groups [groups, R]."""
+    R = W.shape[0]
+    if qmode == "channel":
+        return (W.abs().amax(1) / 7).contiguous(), None
+    if qmode == "static":
+        return (torch.from_numpy(r.uniform(0.2, 0.6, ((C + 63) // 64, R)).astype(np.float32)).to(DEV),
+                (torch.arange(C, device=DEV) // 64).to(torch.int32))
+    return None, None
+
+
+QMODES = {"channel": nat.RQ_QMODE_CHANNEL, "static": nat.RQ_QMODE_STATIC, "dynamic": nat.RQ_QMODE_DYNAMIC}
+
+
+@pytest.mark.parametrize("qmode", ["channel", "static", "dynamic"])
+@pytest.mark.parametrize("count", [128, 40, 20])
+@pytest.mark.parametrize("gmode,terms,sos", [(0, False, 1.0), (0, True, 1.0), (1, True, 1.0), (2, True, 1.0),
+                                             (3, False, 0.7), (3, True, 0.7)])
+def test_quant_block_second_pass(qmode, count, gmode, terms, sos):
+    """The column loop's second pass (IEEE divides, the rows loaded again) in every mode: a block with
+    three rows scaled by 2^70, which sends them and the rows of their waves there, against the same
+    block unscaled, which runs on residual divides alone.  Codes, errors and dynamic scales equal but
+    for the factor (no tolerance)."""
+    r = rng(300 + count + gmode)
+    R, C = 40, 3 * 64
+    i1 = 32
+    def rand(*shape, f=1.0):
+        return torch.from_numpy(r.standard_normal(shape).astype(np.float32) * np.float32(f)).to(DEV)
+    U = torch.triu(rand(C, C, f=0.05))
+    U.diagonal().copy_(torch.from_numpy(r.uniform(0.5, 2.0, C).astype(np.float32)))
+    W, GH, Z = rand(R, C), rand(R, C, f=1e-3), rand(R, C, f=1e-3)
+    anchor = W + rand(R, C, f=1e-2)
+    beta = torch.from_numpy(r.uniform(0, 0.5, R).astype(np.float32)).to(DEV)
+    scale, col_group = _grid_steps(qmode, W, C, r)
+    flag = torch.full((1,), int(terms), dtype=torch.int32, device=DEV)
+    got = []
+    for f in (1.0, WIDE):
+        k = torch.ones((R, 1), device=DEV)
+        k[WIDE_ROWS] = f
+        sc = None if scale is None else (scale * (k.flatten() if qmode == "channel" else k.t())).contiguous()
+        dyn = torch.zeros(R, device=DEV) if qmode == "dynamic" else None
+        codes = torch.zeros((R, C), dtype=torch.int16, device=DEV)
+        err = torch.zeros((R, count), device=DEV)
+        surr = gmode in (1, 2)
+        K.quant_block(W * k, U[None].contiguous(), GH * k, Z * k, R, i1, count, QMODES[qmode], sc, col_group, dyn, 7,
+                      False, False, flag, codes, err, gmode, anchor * k if surr else None, beta if surr else None, sos)
+        torch.cuda.synchronize()
+        got.append((codes, err / k, torch.zeros(1) if dyn is None else dyn / k.flatten()))
+    assert int(got[0][0].ne(0).sum()) > 0.5 * R * count
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("C,B", [(128 * 3 + 40, 128), (32 * 5 + 12, 32)])
+@pytest.mark.parametrize("qmode", ["channel", "static", "dynamic"])
+def test_block_loop_second_pass(qmode, C, B):
+    """The same through rq_block_loop: in the look-ahead launches the second pass loads the weights that
+    its workgroup has just updated.  Codes, dynamic scales and the working weight."""
+    r = rng(400 + C)
+    R = 40
+    Hinv = torch.empty(1, C, C, device=DEV)
+    Hs = _spd(410, C).to(DEV)[None].contiguous()
+    assert K.chol_hinv_attempt(Hs, [0.01], K.chol_workspace(C, DEV, 1), Hinv).tolist() == [0]
+    W = torch.from_numpy(r.standard_normal((R, C)).astype(np.float32)).to(DEV)
+    scale, col_group = _grid_steps(qmode, W, C, r)
+    got = []
+    for f in (1.0, WIDE):
+        k = torch.ones((R, 1), device=DEV)
+        k[WIDE_ROWS] = f
+        sc = None if scale is None else (scale * (k.flatten() if qmode == "channel" else k.t())).contiguous()
+        dyn = torch.zeros((-(-C // B), R), device=DEV) if qmode == "dynamic" else None
+        Wk, codes = W * k, torch.zeros((R, C), dtype=torch.int16, device=DEV)
+        K.block_loop(Wk, Hinv, R, B, QMODES[qmode], sc, col_group, dyn, 7, False, False, codes)
+        torch.cuda.synchronize()
+        got.append((codes, Wk / k, torch.zeros(1) if dyn is None else dyn / k.t()))
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+
+
 @pytest.mark.parametrize("G,R_s,C,B,qmode,atomic", [
-    (2, 150, 128 * 11 + 40, 128, "channel", False),   # two whole groups, far columns spread, ragged last block
-    (1, 40, 128 * 9, 128, "static", True),            # far columns of the second window only
-    (3, 136, 128 * 4, 128, "dynamic", False),         # one group, no far columns
-    (2, 64, 32 * 21 + 4, 32, "channel", False),       # narrow blocks: windows of 160 columns
-    (1, 300, 96 * 13, 96, "dynamic", True),           # windows off the tile grid
-    (2, 48, 64 * 18 + 8, 64, "static", False),
-    (2, 24, 24 * 7 + 4, 24, "channel", False),        # blocks that are not grouped
+    (2, 150, 128 * 11 + 40, 128, "channel", False),   # ragged last block, ragged row tiles
+    (1, 40, 128 * 9, 128, "static", True),            # whole blocks, the last one not atomic
+    (3, 136, 128 * 4, 128, "dynamic", False),
+    (2, 64, 32 * 21 + 4, 32, "channel", False),       # blocks of the narrow column loop, a last one of 4 columns
+    (1, 300, 96 * 13, 96, "dynamic", True),           # blocks off the update's 128-column tiles
+    (2, 48, 64 * 18 + 8, 64, "static", False),        # a last block in the narrow loop, the others not
+    (2, 24, 24 * 7 + 4, 24, "channel", False),
+    (2, 32, 128 + 64, 128, "channel", False),         # two blocks: no column is left for the tiles
     (1, 17, 100, 128, "channel", True),               # one block
     (1, 17, 101, 128, "static", False),
 ])
 def test_block_loop_equals_two_calls(G, R_s, C, B, qmode, atomic):
-    """rq_block_loop (updates of far columns made for four blocks at a time) against rq_quant_block +
-    rq_trailing_update for every block: codes, dynamic scales and the working weight bit for bit."""
+    """rq_block_loop (one launch for the first block, then a look-ahead launch per block with err
+    alternating between two halves of its rows) against rq_quant_block + rq_trailing_update for every
+    block: codes, dynamic scales and the working weight bit for bit."""
     r = rng(170 + C + B)
     R = G * R_s
     Hs = torch.stack([_spd(180 + g, C) for g in range(G)]).to(DEV).contiguous()
