@@ -698,7 +698,8 @@ def traffic_report(fetch_csv, write_csv, cal_fetch_csv, cal_write_csv, kernel_pr
         vals = [float(r["Counter_Value"]) for r in csv.DictReader(open(path))
                 if r["Counter_Name"] == counter and pred(r["Kernel_Name"])]
         return sum(vals) / max(calls or len(vals), 1), len(vals)
-    is_k = lambda n: kernel_prefix in n
+    # (the split kernels' partial tiles are added by a kernel of their own, part of the call)
+    is_k = lambda n: kernel_prefix in n or (kernel_prefix == "k_hessian_split" and "k_split_reduce" in n)
     is_copy = lambda n: "copyBuffer" in n
     # per add_batch call (one profiled step: hessian_calls(cfg) calls, each one or more dispatches)
     ncalls = hessian_calls(cfg)

@@ -909,7 +909,7 @@ __device__ __forceinline__ void whole_or_tail(F&& tile, int logical, int w, cons
 
 // One launch covers a segment of the item list: its `segn` whole items from list position seg0
 // on (od_seg of them off-diagonal), dealt to the XCDs as item_position describes, followed in the
-// last segment by the tail's token slices (the list's items from `full` on).
+// last segment by the tail's ranges and slices (TailPlan; the list's items from `full` on).
 template <typename TX, int PC>
 __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split(
     const uint16_t* __restrict__ XB, int C, const float* __restrict__ sT, int64_t lds_stride,
@@ -925,8 +925,7 @@ __global__ __launch_bounds__(XTHREADS, 1) void k_hessian_split(
   __shared__ __attribute__((aligned(16))) uint8_t lds7[XSTAGE];
   static_assert(XDEPTH == 8, "stage arrays");
   const XStages L{{lds0, lds1, lds2, lds3, lds4, lds5, lds6, lds7}};
-  // Same schedule as k_hessian_accum: XCD-aware order for whole items, then the token
-  // slices of the tail items.
+  // XCD-aware order for the whole items, then the tail's workgroups.
   const int total = ntiles * ntarg;
   const int b = blockIdx.x;
   auto tile = [&](int logical, int64_t kbeg, int64_t kend, float* part) __attribute__((always_inline)) {

@@ -313,7 +313,8 @@ def quant_block(Wp, Hinv_all, GH, Z, R_s, i1, count, qmode, scale, col_group, dy
 def quant_block_lookahead(Wp, Hinv_all, R_s, i1, count, err, count_next, qmode, scale, col_group, dyn_scale,
                           maxq, sym, atomic, codes, err_next):
     """Block k's trailing update (W-only: frozen mode, Z identically zero) and block k+1's
-    quantisation in one launch; equal bit for bit to trailing_update(k) then quant_block(k+1)."""
+    quantisation in one launch; equal bit for bit to trailing_update(k) then quant_block(k+1).  For
+    callers that go block by block; fasterquant runs all its blocks in block_loop."""
     R, C = Wp.shape
     if Hinv_all.shape != (R // R_s, C, C) or not Hinv_all.is_contiguous():
         raise ValueError("quant_block_lookahead: Hinv_all must be contiguous [G, C, C]")

@@ -243,8 +243,9 @@ int rq_trailing_update(float* Wp, int64_t ldw, float* GH, const float* Z, int64_
  * the columns past block k+1 meanwhile.  Writes block k+1's codes and its err to err_next
  * ([R, count_next], a different buffer from err); dyn_scale is block k+1's, atomic applies
  * to block k+1.  Needs count % 8 == 0, C % 4 == 0, (i1 + count + count_next) % 4 == 0 and
- * Hinv_all, err 16-byte aligned (else RQ_EINVAL: use the two calls).  No single counterpart in
- * the reference: it fuses two of its steps for the look-ahead over blocks. */
+ * Hinv_all, err 16-byte aligned (else RQ_EINVAL: use the two calls).  For callers that go block by
+ * block (fasterquant runs all its blocks in rq_block_loop).  No single counterpart in the
+ * reference: it fuses two of its steps for the look-ahead over blocks. */
 int rq_quant_block_lookahead(float* Wp, int64_t ldw, const float* Hinv_all, int C, int R, int R_s,
                              int i1, int count, const float* err, int count_next, int qmode,
                              const float* scale, const int32_t* col_group, float* dyn_scale,
@@ -255,9 +256,9 @@ int rq_quant_block_lookahead(float* Wp, int64_t ldw, const float* Hinv_all, int 
  * with the GPTQ+ terms identically zero: rq_quant_block and rq_trailing_update for every block of
  * blocksize columns, bit for bit, in one launch per block (block k+1 is quantised while block
  * k's update runs, rq_quant_block_lookahead).  codes [R, C]; dyn_scale [blocks, R]
- * (RQ_QMODE_DYNAMIC); err: workspace [R, lde] with lde >= 2 * blocksize, lde % 4 == 0.  atomic: every block but one that ends at C.  More than one
- * block needs blocksize % 8 == 0, C % 4 == 0 and Hinv_all, err 16-byte aligned (else RQ_EINVAL:
- * use the two calls). */
+ * (RQ_QMODE_DYNAMIC); err: workspace [R, lde] with lde >= 2 * blocksize, lde % 4 == 0.  atomic:
+ * every block but one that ends at C.  More than one block needs blocksize % 8 == 0, C % 4 == 0 and
+ * Hinv_all, err 16-byte aligned (else RQ_EINVAL: use the two calls). */
 int rq_block_loop(float* Wp, int64_t ldw, const float* Hinv_all, int C, int R, int R_s, int blocksize,
                   int qmode, const float* scale, const int32_t* col_group, float* dyn_scale, int maxq,
                   int sym, int atomic, int16_t* codes, float* err, int64_t lde, void* stream);
