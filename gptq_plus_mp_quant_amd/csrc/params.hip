@@ -88,8 +88,8 @@ __global__ __launch_bounds__(256) void k_find_params(const TW* __restrict__ w, i
 //    barrier.  Up to MSE_WIDE elements a wave owns one (row, group); wider rows share a
 //    workgroup's 4 waves, which take every fourth batch.
 // 1024 x 4096 fp32 against one 256-thread workgroup per (row, group), every candidate, the IEEE
-// divide and powf: symmetric 16.3 -> 0.40 ms (128-column groups) and 10.7 -> 0.34 ms (per row),
-// asymmetric 16.5 -> 4.1 and 10.5 -> 3.1 ms (of which the sums by powf 3 to 5 %).
+// divide and powf: symmetric 16.3 -> 0.40 ms (128-column groups) and 10.7 -> 0.36 ms (per row),
+// asymmetric 16.5 -> 4.1 and 10.5 -> 3.1 ms (of which the sums by powf 3 to 5 %, of symmetric rows 14 %).
 constexpr int MSE_WIDE = 1024;          // above: one (row, group) per workgroup
 constexpr int MSE_LDS_MAX = 16384;      // elements staged in LDS; wider groups are read in place
 constexpr int MSE_B = 8;                // candidates per batch
@@ -132,18 +132,19 @@ __device__ __forceinline__ float mse_pow(float d, double p, const MseLog* tab) {
 __host__ __device__ constexpr bool mse_distinct(int grid, int steps) { return steps - 1 <= grid; }
 
 // The step and zero of candidate c, and whether it is one of the grid's.  Distinct steps of a
-// symmetric grid (`distinct`, factors that fall from 1 and stay non-negative): c < steps is |xmin|
+// symmetric grid (DISTINCT, factors that fall from 1 and stay non-negative): c < steps is |xmin|
 // shrunk by row c of the grid (where some column leaves xmax no larger), the others xmax shrunk by
-// column c - steps.  Else candidate c is row c / steps, column c % steps.
+// column c - steps.  Else candidate c is row c / steps, column c % steps.  (DISTINCT at run time:
+// 2 % longer, 17 scalar registers more spilled.)
+template <bool SYM, bool DISTINCT>
 struct MseGrid {
   float xmin, xmax, maxq;
-  int sym, grid, steps, n;
-  bool distinct;
+  int grid, steps, n;
   __device__ __forceinline__ float fac(int i) const { return (float)(1.0 - (double)i / (double)grid); }
   __device__ __forceinline__ float lo(int i) const { return fabsf(fac(i) * xmin); }
   __device__ __forceinline__ float hi(int j) const { return fac(j) * xmax; }
   __device__ __forceinline__ bool params(int c, float* s, float* z) const {
-    if (distinct) {
+    if (DISTINCT) {
       const int k = c < steps ? c : c - steps;
       const float m = c < steps ? lo(k) : hi(k);
       // the other side's smallest value decides whether max() ever takes m
@@ -154,7 +155,7 @@ struct MseGrid {
       return c < n && !(other > m) && !(c >= steps && lo(k) == m);
     }
     const float xmin1 = fac(c / steps) * xmin, xmax1 = fac(c % steps) * xmax;
-    if (sym) {
+    if (SYM) {
       *s = rq_clamp_min(rq_nan_max(fabsf(xmin1), xmax1), 1e-5f) / maxq;
       *z = 0.0f;
       return c < n;
@@ -165,7 +166,7 @@ struct MseGrid {
   }
   // place of candidate c in the search order (row by row), for equal errors
   __device__ int64_t first(int c) const {
-    if (!distinct) return c;
+    if (!DISTINCT) return c;
     const bool row = c < steps;
     const int k = row ? c : c - steps;
     const float m = row ? lo(k) : hi(k);
@@ -235,7 +236,7 @@ __device__ __attribute__((noinline)) float mse_any(const TX* x, int n, int lane,
   return (sum[0] + sum[2]) + (sum[1] + sum[3]);
 }
 
-template <bool SYM, typename TW, bool STAGED>
+template <bool SYM, bool DISTINCT, typename TW, bool STAGED>
 __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ w, int R, int C,
                                                          int64_t ldw, int gs, int ng, float maxq,
                                                          int clip_zero, float norm, int grid, int steps,
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
   }
   rmin = __shfl(rmin, 0, 64);
   rmax = __shfl(rmax, 0, 64);
-  MseGrid g;
+  MseGrid<SYM, DISTINCT> g;
   g.xmin = clip_zero ? rq_nan_min(rmin, 0.0f) : rmin;
   g.xmax = clip_zero ? rq_nan_max(rmax, 0.0f) : rmax;
   if (!SYM && g.xmin == 0.0f && g.xmax == 0.0f) {
@@ -294,13 +295,11 @@ __global__ __launch_bounds__(256) void k_find_params_mse(const TW* __restrict__ 
     g.xmax = 1.0f;
   }
   g.maxq = maxq;
-  g.sym = SYM;
   g.grid = grid;
   g.steps = steps;
-  g.distinct = SYM && mse_distinct(grid, steps);
-  g.n = !live ? 0 : g.distinct ? 2 * steps : steps * steps;
+  g.n = !live ? 0 : DISTINCT ? 2 * steps : steps * steps;
   // one step only, the start's (its lower bound), or no error at all: the first candidate wins
-  if (g.distinct && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
+  if (DISTINCT && rq_nan_max(fabsf(g.xmin), g.xmax) <= 1e-5f) g.n = 0;
   if (!SYM && rmin == 0.0f && rmax == 0.0f) g.n = min(g.n, 1);
   const double p = (double)norm;
   const bool fast = norm > 0.0f && norm < 64.0f;
@@ -791,18 +790,21 @@ int launch_find_params_mse(const TW* w, int R, int C, int64_t ldw, int gs, int n
   const int width = gs < C ? gs : C;
   const int per_wg = width <= MSE_WIDE ? 4 : 1;
   const int64_t items = (int64_t)R * ng, wgs = (items + per_wg - 1) / per_wg;
+  const bool distinct = sym && mse_distinct(grid, steps);
   // candidates are counted in 32 bits (46340^2 < 2^31)
-  if (wgs > 0x7fffffff || steps > (sym && mse_distinct(grid, steps) ? 1 << 29 : 46340)) return RQ_EINVAL;
+  if (wgs > 0x7fffffff || steps > (distinct ? 1 << 29 : 46340)) return RQ_EINVAL;
   const bool staged = width <= MSE_LDS_MAX;
   const size_t lds = staged ? (size_t)per_wg * width * sizeof(float) : 0;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), lds, s, w, R, C, ldw, width, ng, (float)maxq, clip_zero,
                        norm, grid, steps, per_wg, scale, zero);
   };
-  if (sym && staged) go(k_find_params_mse<true, TW, true>);
-  else if (sym) go(k_find_params_mse<true, TW, false>);
-  else if (staged) go(k_find_params_mse<false, TW, true>);
-  else go(k_find_params_mse<false, TW, false>);
+  if (distinct && staged) go(k_find_params_mse<true, true, TW, true>);
+  else if (distinct) go(k_find_params_mse<true, true, TW, false>);
+  else if (sym && staged) go(k_find_params_mse<true, false, TW, true>);
+  else if (sym) go(k_find_params_mse<true, false, TW, false>);
+  else if (staged) go(k_find_params_mse<false, false, TW, true>);
+  else go(k_find_params_mse<false, false, TW, false>);
   RQ_CHECK_LAUNCH();
   return RQ_OK;
 }
